@@ -109,7 +109,9 @@ int fwd_views(const DevPlan& P, bool weighted, int tuned, bool prebuilt) {
 // `scratch` names the host-side stand-in of the array; its device address on a GPU comes
 // from hipGetSymbolAddress with that GPU current (resolve_scratch, called when a plan is
 // created on the device) and is the only form in which host code passes it on.
-constexpr size_t kScratchBytes = CTLIB_NOALLOC_SCRATCH_BYTES;
+// Past the advertised size it holds the chunk that the bin tables' copies may read beyond the last row
+// (table_bytes), so that every batch whose data fits the advertised size is served.
+constexpr size_t kScratchBytes = CTLIB_NOALLOC_SCRATCH_BYTES + 2048;
 constexpr int kMaxDevices = 64;
 std::mutex g_scr_mu;
 void* g_scr_ptr[kMaxDevices] = {};
@@ -117,7 +119,7 @@ bool g_scr_tried[kMaxDevices] = {};
 
 }  // namespace
 
-static __device__ __align__(256) unsigned char scratch[CTLIB_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace {
 
@@ -157,19 +159,37 @@ void to_geom(const ctlib_geom* in, Geom* g) {
     g->binshift = in->binshift;
 }
 
-// View chunks of the bin -> pixel launch for a batch of B.  Each (image, line tile) work
-// item's views are split and the partial images summed afterwards, so that the launch
-// has about 4096 blocks: fewer leave CUs idle or badly balanced at the end (measured on
-// 512^2 images: batch 1 runs 5x faster with 12 chunks, batch 32 5% faster with 2).
-// A chunk costs a partial image of traffic and a fixed per-block set-up of about 16
-// views' work, so chunks keep at least 16 views of each axis and there are at most 12.
-int adj_chunks(const ctlib_plan* p, const Tuning& T, int64_t B) {
+// View chunks of the bin -> pixel launch for a batch of B.  The views of each work item (a tile of
+// lines of a group of slices) are split and the partial images summed afterwards, so that the launch
+// fills the chip: counted in tiles of adj_tile_lines lines of one slice, about 4096 (measured on 512^2
+// images: batch 1 runs 5x faster with 12 chunks, batch 32 5% faster with 2).  A chunk costs a partial
+// image of traffic and a fixed per-block set-up of about 16 views' work, so chunks keep at least 16
+// views of each axis and there are at most 12.  The count does not depend on how the kernel groups
+// slices and lines: partial images are rounded to the data type, so it is part of the result.
+// Weighted (its launch shape sh known, whose blocks do twice the work of an edge): the count with the
+// least rounds of resident blocks x (views per chunk + 16) instead; fbp at fan-ED 512^2, B=8: 0.74 ms
+// with 1 chunk against 0.82 with the 8 of the rule above.
+int adj_chunks(const ctlib_plan* p, const Tuning& T, int64_t B, bool weighted, const AdjShape& sh) {
     const DevPlan& P = p->dev;
     int vmin = 1 << 30;
     if (P.nx) vmin = P.nx;
     if (P.ny && P.ny < vmin) vmin = P.ny;
     if (vmin == 1 << 30) return 1;
     if (T.adj_nch > 0) return T.adj_nch < vmin ? T.adj_nch : vmin;
+    if (weighted) {
+        const int vmax = P.nx > P.ny ? P.nx : P.ny;
+        const int64_t blocks = adj_items(P, sh, B), at_once = adj_resident(sh);
+        int best = 1;
+        double least = 0;
+        for (int k = 1; k <= 12 && (k == 1 || k <= vmin / 16); k++) {
+            const double cost = (double)((blocks * k + at_once - 1) / at_once) * ((double)vmax / k + 16);
+            if (k == 1 || cost < least) {
+                least = cost;
+                best = k;
+            }
+        }
+        return best;
+    }
     const int L = adj_tile_lines(P);
     const int64_t items = B * ((P.nx ? (P.H + L - 1) / L : 0) + (P.ny ? (P.W + L - 1) / L : 0));
     int64_t nch = (4096 + items - 1) / items;
@@ -197,11 +217,15 @@ int fwd_chunks(const ctlib_plan* p, const Tuning& T, int64_t B, bool weighted) {
     return nch < 1 ? 1 : (int)nch;
 }
 
+// Bin tables of a batch, and one 64-entry chunk more: the bin -> pixel kernel copies whole chunks.
+size_t table_bytes(const DevPlan& P, int64_t B) { return ((size_t)B * P.V * (P.D + 2) + 64) * sizeof(double2); }
+
 // Scratch layout of every op (byte offsets into ws).
 struct WsLayout {
     size_t ylines = 0, tables = 0, yt = 0, xp = 0, sp = 0, rows = 0, ltab = 0, total = 0;
     size_t n_ylines = 0, n_tables = 0, n_yt = 0, n_xp = 0, n_sp = 0, n_rows = 0, n_ltab = 0;
     int nch = 1;   // view chunks of the bin -> pixel launch (partials in xp / yt when > 1)
+    AdjShape adj{};  // its launch shape, nch included
     int fnch = 1;  // line chunks of the line -> bin launch (partial sinograms in sp when > 1)
     int fwd_G = 0; // views per line -> bin block override (Tuning::fwd_G)
 
@@ -220,8 +244,9 @@ WsLayout layout(const ctlib_plan* p, const Tuning& T, int op, int64_t B, int dty
         L.fnch = fwd_chunks(p, T, B, weighted);
         L.n_sp = L.fnch > 1 ? L.fnch * sino * es : 0;
     };
-    auto partials = [&]() {
-        L.nch = adj_chunks(p, T, B);
+    auto partials = [&](bool weighted) {
+        L.adj = adj_shape(P, dtype == CTLIB_F64 ? DT_F64 : DT_F32, weighted, B);
+        L.nch = L.adj.nch = adj_chunks(p, T, B, weighted, L.adj);
         L.n_yt = P.ny ? L.nch * img * es : 0;
         L.n_xp = (L.nch > 1 && P.nx) ? L.nch * img * es : 0;
     };
@@ -235,13 +260,13 @@ WsLayout layout(const ctlib_plan* p, const Tuning& T, int op, int64_t B, int dty
         break;
     case CTLIB_OP_PRJ_T:
     case CTLIB_OP_BPRJ:
-        L.n_tables = (size_t)B * P.V * (P.D + 2) * sizeof(double2);
-        partials();
+        L.n_tables = table_bytes(P, B);
+        partials(op == CTLIB_OP_BPRJ);
         break;
     case CTLIB_OP_FBP:
         L.n_rows = sino * sizeof(double);
-        L.n_tables = (size_t)B * P.V * (P.D + 2) * sizeof(double2);
-        partials();
+        L.n_tables = table_bytes(P, B);
+        partials(true);
         break;
     case CTLIB_OP_FBP_T:
         L.n_ylines = P.ny ? img * es : 0;
@@ -249,7 +274,7 @@ WsLayout layout(const ctlib_plan* p, const Tuning& T, int op, int64_t B, int dty
         sino_partials(true);
         break;
     case CTLIB_OP_BPRJ_SV:
-        L.n_tables = (size_t)B * P.V * (P.D + 2) * sizeof(double2);
+        L.n_tables = table_bytes(P, B);
         break;
     default:
         break;
@@ -398,7 +423,7 @@ hipError_t run_to_image(const ctlib_plan* p, int dtype, const double2* tabs, voi
     hipError_t e;
     {
         KernelTimer t(K_ADJ, sweep_bytes(P, B, dtype), 0, s);
-        e = launch_adj(P, dtype, tabs, outX, yt, B, weighted, wscale, AdjShape{L.nch}, s);
+        e = launch_adj(P, dtype, tabs, outX, yt, B, weighted, wscale, L.adj, s);
     }
     if (e != hipSuccess) return e;
     KernelTimer t(K_AUX, 0, 0, s);
@@ -832,7 +857,7 @@ ResidLayout resid_layout(const ctlib_plan* p, const Tuning& T, int64_t batch, in
     R.la = layout(p, T, CTLIB_OP_PRJ, batch, dtype);
     R.lb = layout(p, T, CTLIB_OP_PRJ_T, batch, dtype);
     R.tables = R.la.total > R.lb.total ? R.la.total : R.lb.total;
-    R.total = R.tables + align_up((size_t)batch * p->dev.V * (p->dev.D + 2) * sizeof(double2));
+    R.total = R.tables + align_up(table_bytes(p->dev, batch));
     return R;
 }
 

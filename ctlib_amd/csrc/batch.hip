@@ -110,12 +110,12 @@ __device__ __forceinline__ void run_adj_geo(const SliceDev& sd, int mode, int ti
     T* ox = (T*)sd.grad;
     T* oy = (T*)sd.yt;
     switch (sd.acls & 3) {
-    case GEO_ED: adj_block<T, LPW, NPE, false, GEO_ED, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, 1.0, smem); break;
-    case GEO_EA: adj_block<T, LPW, NPE, false, GEO_EA, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, 1.0, smem); break;
+    case GEO_ED: adj_block<T, LPW, NPE, GEO_ED, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, smem); break;
+    case GEO_EA: adj_block<T, LPW, NPE, GEO_EA, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, smem); break;
     case GEO_PARA:
-        adj_block<T, LPW, NPE, false, GEO_PARA, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, 1.0, smem);
+        adj_block<T, LPW, NPE, GEO_PARA, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, smem);
         break;
-    default: adj_block<T, LPW, NPE, false, GEO_EAP, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, 1.0, smem); break;
+    default: adj_block<T, LPW, NPE, GEO_EAP, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, smem); break;
     }
 }
 

@@ -1,12 +1,12 @@
-// Stand-alone launches of the bin -> pixel kernels (gfx950): projection_t and
-// backprojection (k_adj) and the per-view backprojection_sv (k_bprj_sv).  The
-// per-work-item device code lives in dd_device.h; kept apart from the line ->
-// bin launches so the two translation units compile in parallel.
+// Launch shapes of the bin -> pixel kernels (projection_t and backprojection; k_adj in
+// dd_adj_group.h, compiled per data type and weighting in dd_adj_f32.hip, dd_adj_w_f32.hip,
+// dd_adj_f64.hip and dd_adj_w_f64.hip so that they build in parallel), the sum of their partial
+// images and the per-view backprojection_sv (k_bprj_sv).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 
-#include "dd_device.h"
+#include "dd_adj_group.h"
 #include "kernels.h"
 
 namespace ctlib {
@@ -14,30 +14,6 @@ namespace ctlib {
 using namespace dd;
 
 namespace {
-
-// One launch covers both sweep axes: work items [0, B*ntx) are (b, tile of
-// 4*LPW image rows) over the X-axis views, the rest (b, tile of columns) over
-// the Y-axis views, written bottom-to-top to outYT.  With nch > 1 every item is
-// split into nch chunks of its axis's views; chunk k writes its partial image
-// k*B*H*W elements into outX / outYT.
-template <typename T, int LPW, int NPE, bool WEIGHTED, int GEO, bool EXACT>
-__global__ __launch_bounds__(256) void k_adj(DevPlan P, const double2* __restrict__ tabs, T* __restrict__ outX,
-                                             T* __restrict__ outYT, int B, int ntx, int nty, double wscale, int nch) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int nwx = B * ntx;
-    int w = xcd_remap(blockIdx.x, gridDim.x, (nwx + B * nty) * nch);
-    if (w < 0) return;
-    const int ch = w % nch;
-    w /= nch;
-    const int mode = w < nwx ? MODE_X : MODE_Y;
-    if (mode == MODE_Y) w -= nwx;
-    const int ntiles = mode == MODE_Y ? nty : ntx;
-    const int b = w / ntiles, tile = w - b * ntiles;
-    const int nv = mode == MODE_Y ? P.ny : P.nx;
-    const size_t part = (size_t)ch * B * P.H * P.W;
-    adj_block<T, LPW, NPE, WEIGHTED, GEO, EXACT>(P, tabs, outX + part, outYT + part, b, mode, tile, wscale, smem,
-                                                 ch * nv / nch, (ch + 1) * nv / nch);
-}
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_combine_parts(T* __restrict__ out, const T* __restrict__ xs,
@@ -235,61 +211,46 @@ __global__ __launch_bounds__(256) void k_bprj_sv(DevPlan P, const double2* __res
 
 namespace {
 
-template <typename T, int LPW, int NPE, bool WTD, int GEO, bool EXACT>
-hipError_t adj_launch_t(const DevPlan& P, const double2* tabs, void* outX, void* outYT, int B, double wscale,
-                        int nch, hipStream_t s) {
-    const int L = 4 * LPW;
-    const int ntx = P.nx ? (P.H + L - 1) / L : 0;
-    const int nty = P.ny ? (P.W + L - 1) / L : 0;
-    const long long nw = (long long)(ntx + nty) * B * nch;
-    if (nw > (1LL << 30)) return hipErrorInvalidValue;  // grid size (one block per work item)
-    const int nwork = (int)nw;
-    const size_t lds = adj_block_lds(P.D, L);
-    auto kern = k_adj<T, LPW, NPE, WTD, GEO, EXACT>;
-    if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(kern, dim3(grid_for(nwork)), dim3(NT), lds, s, P, tabs, (T*)outX, (T*)outYT, B, ntx, nty,
-                       wscale, nch);
-    return hipGetLastError();
+template <typename T, int NS, bool WEIGHTED>
+bool shape_for(const DevPlan& P, AdjShape* sh) {
+    const int n = P.ny && P.H > (P.nx ? P.W : 0) ? P.H : P.W;
+    const int most = adjg_most<T, NS, WEIGHTED>(P.scan_type == GEO_EA), waves = adjg_waves<T, NS, WEIGHTED>();
+    sh->NS = NS;
+    sh->PH = 1;
+    while (32 * most * sh->PH < n) sh->PH *= 2;
+    if (sh->PH > waves) return false;
+    sh->SL = (n + 32 * sh->PH - 1) / (32 * sh->PH);
+    if (sh->SL < 4) sh->SL = 4;
+    while (!adjg_has_slots(most, sh->SL)) sh->SL++;
+    sh->L = 2 * (waves / sh->PH);
+    sh->nch = 1;
+    return true;
 }
 
-template <typename T, bool WTD, int GEO>
-hipError_t adj_npe(const DevPlan& P, const double2* tabs, void* outX, void* outYT, int B, double wscale, int nch,
-                   hipStream_t s) {
-    int n = P.nx ? P.W : 0;
-    if (P.ny && P.H > n) n = P.H;
-    const int npe = (n + 1 + 63) / 64;
-    // every line (rows of X views, columns of Y views) exactly 64 * (NPE - 1) pixels
-    auto exact = [&](int NPE) { return (P.nx == 0 || P.W == 64 * (NPE - 1)) && (P.ny == 0 || P.H == 64 * (NPE - 1)); };
-    if (npe <= 5) return exact(5) ? adj_launch_t<T, 8, 5, WTD, GEO, true>(P, tabs, outX, outYT, B, wscale, nch, s)
-                                  : adj_launch_t<T, 8, 5, WTD, GEO, false>(P, tabs, outX, outYT, B, wscale, nch, s);
-    if (npe <= 7) return exact(7) ? adj_launch_t<T, 4, 7, WTD, GEO, true>(P, tabs, outX, outYT, B, wscale, nch, s)
-                                  : adj_launch_t<T, 4, 7, WTD, GEO, false>(P, tabs, outX, outYT, B, wscale, nch, s);
-    if (npe <= 9) return exact(9) ? adj_launch_t<T, 4, 9, WTD, GEO, true>(P, tabs, outX, outYT, B, wscale, nch, s)
-                                  : adj_launch_t<T, 4, 9, WTD, GEO, false>(P, tabs, outX, outYT, B, wscale, nch, s);
-    if (npe <= 13) return exact(13) ? adj_launch_t<T, 2, 13, WTD, GEO, true>(P, tabs, outX, outYT, B, wscale, nch, s)
-                                    : adj_launch_t<T, 2, 13, WTD, GEO, false>(P, tabs, outX, outYT, B, wscale, nch, s);
-    if (npe <= 17) return exact(17) ? adj_launch_t<T, 2, 17, WTD, GEO, true>(P, tabs, outX, outYT, B, wscale, nch, s)
-                                    : adj_launch_t<T, 2, 17, WTD, GEO, false>(P, tabs, outX, outYT, B, wscale, nch, s);
-    if (npe <= 33) return adj_launch_t<T, 1, 33, WTD, GEO, false>(P, tabs, outX, outYT, B, wscale, nch, s);
-    return hipErrorInvalidValue;
-}
-
-template <typename T, bool WTD>
-hipError_t adj_geo(const DevPlan& P, const double2* tabs, void* outX, void* outYT, int B, double wscale, int nch,
-                   hipStream_t s) {
-    switch (P.scan_type) {
-    case GEO_ED: return adj_npe<T, WTD, GEO_ED>(P, tabs, outX, outYT, B, wscale, nch, s);
-    case GEO_EA:
-        return P.ea_poly ? adj_npe<T, WTD, GEO_EAP>(P, tabs, outX, outYT, B, wscale, nch, s)
-                         : adj_npe<T, WTD, GEO_EA>(P, tabs, outX, outYT, B, wscale, nch, s);
-    default: return adj_npe<T, WTD, GEO_PARA>(P, tabs, outX, outYT, B, wscale, nch, s);
-    }
+template <typename T, bool WEIGHTED>
+AdjShape shape_of(const DevPlan& P, int64_t B) {
+    // Four slices share one lookup from batch 3 on (a block of four costs less than two of two even
+    // with a slice repeated), if four double-buffered tables fit the LDS (1022 bins); else two.
+    AdjShape sh{};
+    if (B >= 3 && P.D <= adjg_max_bins<4>() && shape_for<T, 4, WEIGHTED>(P, &sh)) return sh;
+    if (B >= 2 && shape_for<T, 2, WEIGHTED>(P, &sh)) return sh;
+    shape_for<T, 1, WEIGHTED>(P, &sh);
+    return sh;
 }
 
 }  // namespace
+
+AdjShape adj_shape(const DevPlan& P, int dtype, bool weighted, int64_t B) {
+    if (dtype == DT_F32) return weighted ? shape_of<float, true>(P, B) : shape_of<float, false>(P, B);
+    return weighted ? shape_of<double, true>(P, B) : shape_of<double, false>(P, B);
+}
+
+int64_t adj_items(const DevPlan& P, const AdjShape& sh, int64_t B) {
+    return (B + sh.NS - 1) / sh.NS * ((P.nx ? (P.H + sh.L - 1) / sh.L : 0) + (P.ny ? (P.W + sh.L - 1) / sh.L : 0));
+}
+
+// 256 CUs; one block of several slices fills a CU's registers and most of its LDS.
+int adj_resident(const AdjShape& sh) { return sh.NS == 1 ? 512 : 256; }
 
 int adj_tile_lines(const DevPlan& P) {
     int n = P.nx ? P.W : 0;
@@ -316,12 +277,9 @@ hipError_t launch_adj(const DevPlan& P, int dtype, const double2* tabs, void* ou
     if (B <= 0 || P.nx + P.ny == 0) return hipSuccess;
     if (sh.nch < 1) sh.nch = 1;
     if ((P.nx && sh.nch > P.nx) || (P.ny && sh.nch > P.ny)) return hipErrorInvalidValue;
-    if (dtype == DT_F32) {
-        return weighted ? adj_geo<float, true>(P, tabs, outX, outYT, B, wscale, sh.nch, s)
-                        : adj_geo<float, false>(P, tabs, outX, outYT, B, wscale, sh.nch, s);
-    }
-    return weighted ? adj_geo<double, true>(P, tabs, outX, outYT, B, wscale, sh.nch, s)
-                    : adj_geo<double, false>(P, tabs, outX, outYT, B, wscale, sh.nch, s);
+    const AdjArgs a{tabs, outX, outYT, B, wscale, sh};
+    if (dtype == DT_F32) return weighted ? launch_adj_w_f32(P, a, s) : launch_adj_f32(P, a, s);
+    return weighted ? launch_adj_w_f64(P, a, s) : launch_adj_f64(P, a, s);
 }
 
 namespace {

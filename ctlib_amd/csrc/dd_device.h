@@ -60,6 +60,24 @@ __device__ __forceinline__ double rcp_refined(double d) {
     return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
 }
 
+// Asynchronous copy of 16 bytes per active lane, global (uniform `src` + the lane's byte offset) ->
+// LDS (uniform byte address `dst` + 16 * lane), counted in vmcnt.  Written as asm and waited for by hand: after the
+// builtin the compiler holds every LDS read to be unordered with the copy and waits for all of a
+// wave's reads (lgkmcnt(0)) where it needs the oldest, which leaves nothing in flight.  M0 is set here
+// and used by nothing else (a kernel with a builtin that needs M0 must not hold it across this).
+__device__ __forceinline__ void copy_to_lds16(const void* src, unsigned lane_off, unsigned dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(src), "s"(dst)
+                 : "memory");
+}
+// LDS byte address of a shared-memory pointer, uniform.
+__device__ __forceinline__ unsigned lds_address(const void* p) {
+    return __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
+}
+
+// Position of a lane in the order in which the passes of ds_read_b128 take the lanes: passes 0..3
+// hold positions 0-15, 16-31, 32-47, 48-63 (an involution: bit 4 flips where bits 2 and 3 differ).
+__device__ __forceinline__ int b128_pos(int lane) { return lane ^ ((((lane >> 2) ^ (lane >> 3)) & 1) << 4); }
+
 // Index of a cumulative table from a float coordinate, clamped to [0, hi].
 __device__ __forceinline__ int table_index(float q, float hi) { return (int)__builtin_amdgcn_fmed3f(q, 0.0f, hi); }
 
@@ -884,7 +902,7 @@ __device__ __forceinline__ double eval_G_lk(const double2* __restrict__ t, doubl
 
 // LDS bytes of one adj_block.
 __host__ __device__ inline size_t adj_block_lds(int D, int L) {
-    return (size_t)2 * (D + 2) * 16 + (size_t)2 * L * LC_WORDS * 8 + (size_t)4 * L * 16;
+    return (size_t)2 * (D + 2) * 16 + (size_t)2 * L * LC_WORDS * 8 + (size_t)2 * L * 16;
 }
 
 // One bin -> pixel work item: batch element b, sweep axis `mode`, image lines
@@ -898,18 +916,18 @@ __host__ __device__ inline size_t adj_block_lds(int D, int L) {
 // the only edge of group NPE-1; instead of a ninth (or seventeenth) group per
 // line, lane q of the wave evaluates edge n of its line q (LPW <= 64 lanes),
 // one evaluation per view for all the wave's lines.
-// Views [vb, ve) of the axis list (ve < 0: all) contribute; a launch split into
-// view chunks writes each chunk's partial image and sums them afterwards.
-template <typename T, int LPW, int NPE, bool WEIGHTED, int GEO, bool EXACT = false>
+// Used by the batch kernel, whose slices have a geometry each; the stand-alone launches share the
+// lookups of a batch's slices (dd_adj_group.h).
+template <typename T, int LPW, int NPE, int GEO, bool EXACT = false>
 __device__ __forceinline__ void adj_block(const DevPlan& P, const double2* __restrict__ tabs, T* __restrict__ outX,
-                                          T* __restrict__ outYT, int b, int mode, int tile, double wscale,
-                                          unsigned char* __restrict__ smem, int vb = 0, int ve = -1) {
+                                          T* __restrict__ outYT, int b, int mode, int tile,
+                                          unsigned char* __restrict__ smem) {
     constexpr int L = 4 * LPW;
     constexpr int NG = EXACT ? NPE - 1 : NPE;  // edge groups evaluated per line
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int* vlist = mode == MODE_Y ? P.yviews : P.xviews;
-    const int nv = ve < 0 ? (mode == MODE_Y ? P.ny : P.nx) : ve;
+    const int nv = mode == MODE_Y ? P.ny : P.nx;
     const int nlines = mode == MODE_Y ? P.W : P.H;
     const int n = mode == MODE_Y ? P.H : P.W;
     const int D = P.D;
@@ -920,9 +938,7 @@ __device__ __forceinline__ void adj_block(const DevPlan& P, const double2* __res
     double2* stab = reinterpret_cast<double2*>(smem);          // [2][tabn]
     double* scf = reinterpret_cast<double*>(stab + 2 * tabn);  // [2][L][LC_WORDS]
     float4* slk = reinterpret_cast<float4*>(scf + 2 * L * LC_WORDS);  // [2][L] composed lookups (fp32 data)
-    float4* swk = slk + 2 * L;  // [2][L] pre-scaled pixel-weight coefficients (fp32 data, weighted)
     constexpr bool LK = sizeof(T) == 4;
-    constexpr bool WK = WEIGHTED && LK;
 
     const double2* tb_b = tabs + (size_t)b * P.V * tabn;
     // Asynchronous copy of view v's table into LDS buffer `buf`: wave w copies
@@ -949,9 +965,6 @@ __device__ __forceinline__ void adj_block(const DevPlan& P, const double2* __res
     auto lk_word = [&](int v) {
         return athread && al < nlines ? P.adj_lk[(size_t)v * P.max_lines + al] : make_float4(0.f, 0.f, 0.f, 1.f);
     };
-    auto wk_word = [&](int v) {
-        return athread && al < nlines ? P.adj_wk[(size_t)v * P.max_lines + al] : make_float4(0.f, 0.f, 0.f, 1.f);
-    };
 
     // Tiles of 16 or more lines (DMA): the LineCoefs (16 bytes of line tid/4 per thread
     // tid < 4L) and composed lookups (thread tid < L) are copied global -> LDS like the table,
@@ -970,9 +983,6 @@ __device__ __forceinline__ void adj_block(const DevPlan& P, const double2* __res
         if (LK && tid < L)
             __builtin_amdgcn_global_load_lds((const void*)(P.adj_lk + (size_t)v * P.max_lines + min(al, nlines - 1)),
                                              (__attribute__((address_space(3))) void*)(slk + buf * L), 16, 0, 0);
-        if (WK && tid < L)
-            __builtin_amdgcn_global_load_lds((const void*)(P.adj_wk + (size_t)v * P.max_lines + min(al, nlines - 1)),
-                                             (__attribute__((address_space(3))) void*)(swk + buf * L), 16, 0, 0);
     };
     auto view_barrier = [&]() {
         if (DMA) {
@@ -993,21 +1003,20 @@ __device__ __forceinline__ void adj_block(const DevPlan& P, const double2* __res
     double accx = 0.0;                          // EXACT: lane q accumulates edge n of line q
     const int lx = (lane < LPW ? lane : 0) * 4 + wave;  // that line within the tile
 
-    table_to_lds(vlist[vb], 0);
+    table_to_lds(vlist[0], 0);
     if (DMA) {
-        side_to_lds(vlist[vb], 0);
+        side_to_lds(vlist[0], 0);
     } else {
-        if (cthread) scf[tid] = coef_word(vlist[vb]);
-        if (athread) slk[tid] = lk_word(vlist[vb]);
-        if (WK && athread) swk[tid] = wk_word(vlist[vb]);
+        if (cthread) scf[tid] = coef_word(vlist[0]);
+        if (athread) slk[tid] = lk_word(vlist[0]);
     }
     view_barrier();
 
-    for (int iv = vb; iv < nv; iv++) {
-        const int cur = (iv - vb) & 1;
+    for (int iv = 0; iv < nv; iv++) {
+        const int cur = iv & 1;
         const int v = vlist[iv];
         double cnext = 0.0;
-        float4 anext = make_float4(0.f, 0.f, 0.f, 1.f), wnext = anext;
+        float4 anext = make_float4(0.f, 0.f, 0.f, 1.f);
         if (iv + 1 < nv) {
             const int vn = vlist[iv + 1];
             table_to_lds(vn, cur ^ 1);
@@ -1016,19 +1025,13 @@ __device__ __forceinline__ void adj_block(const DevPlan& P, const double2* __res
             } else {
                 cnext = coef_word(vn);
                 if (athread) anext = lk_word(vn);
-                if (WK && athread) wnext = wk_word(vn);
             }
         }
         const double2* t = stab + cur * tabn;
         const double* cf = scf + cur * L * LC_WORDS;
         const float4* clk = slk + cur * L;
-        const float4* cwk = swk + cur * L;
         const Lookup lu = view_lookup(P, v);
-        double gx = 0.0;  // EXACT: G at edge n of line lx (lanes >= LPW: unused)
-        if (EXACT) {
-            gx = eval_G<GEO, sizeof(T) == 8>(t, cf[lx * LC_WORDS + LC_A0], cf[lx * LC_WORDS + LC_S], n, lu, hi);
-            if (!WEIGHTED) accx += gx;
-        }
+        if (EXACT) accx += eval_G<GEO, sizeof(T) == 8>(t, cf[lx * LC_WORDS + LC_A0], cf[lx * LC_WORDS + LC_S], n, lu, hi);
 #pragma unroll
         for (int q = 0; q < LPW; q++) {
             const int lq = q * 4 + wave;  // line within the tile
@@ -1050,59 +1053,11 @@ __device__ __forceinline__ void adj_block(const DevPlan& P, const double2* __res
                     return eval_G<GEO, true>(t, a, s, lane + 64 * i, lu, hi);
                 }
             };
-            if (!WEIGHTED) {
 #pragma unroll
-                for (int i = 0; i < NG; i++) acc[q][i] += G_at(i);
-            } else {
-                // Pixel weight inv_s / ((w0 + w1 p)^2 + w2) of pixel p = lane + 64 k (the call's
-                // scale multiplies the output).  fp32 storage: from the plan's pre-scaled fp32
-                // coefficients, 1 / (u^2 + c^2 w2) with u = k (64 c w1) + u0 (relative error
-                // ~3e-7, below the output's rounding); fp64 storage: u and d in fp64,
-                // Newton-refined reciprocal.
-                const double w0 = cf[lq * LC_WORDS + LC_W0], w1 = cf[lq * LC_WORDS + LC_W1];
-                const double w2 = cf[lq * LC_WORDS + LC_W2];
-                const double ws = cf[lq * LC_WORDS + LC_INVS];
-                float4 wk = make_float4(0.f, 0.f, 0.f, 1.f);
-                if (WK) wk = cwk[lq];
-                const float u0 = __builtin_fmaf(wk.y, (float)lane, wk.z);
-                auto wgt = [&](int k) {
-                    if constexpr (WK) {
-                        const float u = k == 0 ? u0 : __builtin_fmaf((float)k, wk.x, u0);
-                        return (double)__builtin_amdgcn_rcpf(__builtin_fmaf(u, u, wk.w));
-                    } else {
-                        const double u = __builtin_fma(w1, (double)(lane + 64 * k), w0);
-                        const double d = __builtin_fma(u, u, w2);
-                        return ws * rcp_refined(d);
-                    }
-                };
-                // right edge of pixel lane + 64 (i-1): edge lane+1 of group i-1, or for
-                // lane 63 edge 0 of group i; both come from the rotations of the groups
-                double gprev = 0.0, rprev = 0.0;
-#pragma unroll
-                for (int i = 0; i < NG; i++) {
-                    const double gi = G_at(i);
-                    const double ri = rot_next_d(gi);
-                    if (i > 0) {
-                        const double right = lane == 63 ? ri : rprev;
-                        // pixels past the line accumulate unused values (never stored)
-                        acc[q][i - 1] += wgt(i - 1) * (right - gprev);
-                    }
-                    gprev = gi;
-                    rprev = ri;
-                }
-                if (EXACT) {
-                    // last group: lane 63's pixel n-1 ends at edge n, evaluated by lane q
-                    const double gxq = readlane_d(gx, q);
-                    acc[q][NG - 1] += wgt(NG - 1) * ((lane == 63 ? gxq : rprev) - gprev);
-                } else {
-                    // pixels of the last slot group (lane 63's pixel is past the line since 64 * NPE > n)
-                    acc[q][NPE - 1] += wgt(NPE - 1) * (rprev - gprev);
-                }
-            }
+            for (int i = 0; i < NG; i++) acc[q][i] += G_at(i);
         }
         if (!DMA && iv + 1 < nv && cthread) scf[(cur ^ 1) * L * LC_WORDS + tid] = cnext;
         if (!DMA && iv + 1 < nv && athread) slk[(cur ^ 1) * L + tid] = anext;
-        if (!DMA && WK && iv + 1 < nv && athread) swk[(cur ^ 1) * L + tid] = wnext;
         view_barrier();
     }
 
@@ -1116,19 +1071,14 @@ __device__ __forceinline__ void adj_block(const DevPlan& P, const double2* __res
         for (int i = 0; i < NG; i++) {
             if (i >= npe) continue;  // wave-uniform
             const int p = lane + 64 * i;
-            double val;
-            if (!WEIGHTED) {
-                double right = shfl_next_d(acc[q][i]);
-                double r0 = 0.0;
+            double right = shfl_next_d(acc[q][i]);
+            double r0 = 0.0;
 #pragma unroll
-                for (int k = 0; k < NG; k++)
-                    if (k == i + 1) r0 = readlane_d(acc[q][k], 0);
-                if (EXACT && i == NG - 1) r0 = readlane_d(accx, q);
-                if (lane == 63) right = r0;
-                val = right - acc[q][i];
-            } else {
-                val = acc[q][i] * wscale;
-            }
+            for (int k = 0; k < NG; k++)
+                if (k == i + 1) r0 = readlane_d(acc[q][k], 0);
+            if (EXACT && i == NG - 1) r0 = readlane_d(accx, q);
+            if (lane == 63) right = r0;
+            const double val = right - acc[q][i];
             if (p < n) dst[p] = (T)val;
         }
     }

@@ -40,7 +40,20 @@ struct FwdShape {                 // line->bin kernel
     int G;                        // views per block
     int nch;                      // line chunks (<= 1: none)
 };
-struct AdjShape { int nch; };     // view chunks of the bin->pixel kernel (<= 1: none)
+// bin->pixel kernel: NS slices per block, tiles of L lines, SL slots of 32 pixel edges per wave and
+// PH waves along a line (adj_shape); nch view chunks (<= 1: none)
+struct AdjShape {
+    int NS, SL, PH, L;
+    int nch;
+};
+struct AdjArgs {
+    const double2* tabs;
+    void* outX;
+    void* outYT;
+    int B;
+    double wscale;
+    AdjShape sh;
+};
 
 // x [B][H][W] -> xT [B][W][H] with xT[b][c][i] = x[b][H-1-i][c]  (Y-mode lines, bottom to top)
 hipError_t launch_to_ylines(const void* x, void* xT, int dtype, int B, int H, int W, hipStream_t s);
@@ -96,8 +109,17 @@ hipError_t launch_bin_tables(const DevPlan& P, int in_dtype, const void* y, cons
 // writes its partial images at outX + c*B*H*W and outYT + c*B*H*W (elements); launch_combine_parts sums them.
 hipError_t launch_adj(const DevPlan& P, int dtype, const double2* tabs, void* outX, void* outYT, int B,
                       bool weighted, double wscale, AdjShape shape, hipStream_t s);
-// Image lines per work item of launch_adj (work items = B * (ceil(H/L) [X views] + ceil(W/L) [Y views])).
+// Launch shape of launch_adj for a batch of B, without the view chunks (nch = 1).
+AdjShape adj_shape(const DevPlan& P, int dtype, bool weighted, int64_t B);
+// Its work items (slice groups x line tiles of both axes), and the blocks the chip holds at once.
+int64_t adj_items(const DevPlan& P, const AdjShape& sh, int64_t B);
+int adj_resident(const AdjShape& sh);
+// Image lines that the view chunks are counted in (abi.cpp adj_chunks).
 int adj_tile_lines(const DevPlan& P);
+hipError_t launch_adj_f32(const DevPlan& P, const AdjArgs& a, hipStream_t s);
+hipError_t launch_adj_w_f32(const DevPlan& P, const AdjArgs& a, hipStream_t s);
+hipError_t launch_adj_f64(const DevPlan& P, const AdjArgs& a, hipStream_t s);
+hipError_t launch_adj_w_f64(const DevPlan& P, const AdjArgs& a, hipStream_t s);
 // out[b][r][c] = sum_k xs[k][b][r][c] (hasX) + sum_k ys[k][b][c][H-1-r] (hasY), k < nch
 hipError_t launch_combine_parts(void* out, const void* xs, const void* ys, int dtype, int B, int H, int W, int nch,
                                 bool hasX, bool hasY, hipStream_t s);
