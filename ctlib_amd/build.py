@@ -65,6 +65,8 @@ def build(arch="gfx950", verbose=False, with_torch=True):
         "dd_adj.o": [HIPCC, f"--offload-arch={arch}", *HIP_FLAGS, "-c", os.path.join(CSRC, "dd_adj.hip")],
         **{f"dd_adj_{v}.o": [HIPCC, f"--offload-arch={arch}", *HIP_FLAGS, "-c", os.path.join(CSRC, f"dd_adj_{v}.hip")]
            for v in ("f32", "w_f32", "f64", "w_f64")},
+        **{f"dd_fwd_lt_{v}.o": [HIPCC, f"--offload-arch={arch}", *HIP_FLAGS, "-c",
+                                os.path.join(CSRC, f"dd_fwd_lt_{v}.hip")] for v in ("f32", "f64")},
         "dd_fwd_w.o": [HIPCC, f"--offload-arch={arch}", *HIP_FLAGS, "-c", os.path.join(CSRC, "dd_fwd_w.hip")],
         "ramp_mfma.o": [HIPCC, f"--offload-arch={arch}", *HIP_FLAGS, "-c", os.path.join(CSRC, "ramp_mfma.hip")],
         "batch.o": [HIPCC, f"--offload-arch={arch}", *HIP_FLAGS, "-c", os.path.join(CSRC, "batch.hip")],

@@ -66,7 +66,8 @@ __device__ __forceinline__ double rcp_refined(double d) {
 // wave's reads (lgkmcnt(0)) where it needs the oldest, which leaves nothing in flight.  M0 is set here
 // and used by nothing else (a kernel with a builtin that needs M0 must not hold it across this).
 __device__ __forceinline__ void copy_to_lds16(const void* src, unsigned lane_off, unsigned dst) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(src), "s"(dst)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(src),
+                 "s"(__builtin_amdgcn_readfirstlane(dst))
                  : "memory");
 }
 // LDS byte address of a shared-memory pointer, uniform.
@@ -89,6 +90,22 @@ __device__ __forceinline__ int table_index_d(double q, int hi) {
     int j = (int)q, r;
     asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(j), "v"(hi));
     return r;
+}
+
+// The same with a uniform bound.
+__device__ __forceinline__ int table_index_u(double q, int hi) {
+    int j = (int)q, r;
+    asm("v_med3_i32 %0, %1, 0, %2" : "=v"(r) : "v"(j), "s"(hi));
+    return r;
+}
+
+// A uniform pointer in scalar registers, whatever the compiler knows.
+template <typename V>
+__device__ __forceinline__ V* scalar_ptr(V* p) {
+    int2 a = __builtin_bit_cast(int2, p);
+    a.x = __builtin_amdgcn_readfirstlane(a.x);
+    a.y = __builtin_amdgcn_readfirstlane(a.y);
+    return __builtin_bit_cast(V*, a);
 }
 
 __device__ __forceinline__ double readlane_d(double v, int lane) {

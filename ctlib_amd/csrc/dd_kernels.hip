@@ -1,7 +1,7 @@
 // Stand-alone launches of the line -> bin kernels (gfx950): projection,
-// backprojection_t and the residual-fused forward (k_fwd), the per-(slice,
-// view) bin tables of the adjoints, and the Y-axis line copy / combine
-// transposes.  The per-work-item device code lives in dd_device.h; the
+// backprojection_t and the residual-fused forward with the line tables built per block (k_fwd; over
+// prebuilt tables: dd_fwd_group.h), the line tables, the per-(slice, view) bin tables of the adjoints,
+// and the Y-axis line copy / combine transposes.  The per-work-item device code lives in dd_device.h; the
 // persistent heterogeneous batch kernel (batch.hip) runs the same block
 // functions, and the bin -> pixel launches live in dd_adj.hip.
 #include <hip/hip_runtime.h>
@@ -44,30 +44,53 @@ __global__ __launch_bounds__(256) void k_line_tables(DevPlan P, const T* __restr
     line_table_wave<T, M>(row, l < hx ? P.W : P.H, lt + (size_t)line * ltab_n<M>(), threadIdx.x & 63);
 }
 
-// Line-table buffers of k_fwd_lt (one line ahead).
-constexpr int FWD_LT_BUFFERS = 2;
-
-// k_fwd over the prebuilt line tables of k_line_tables (unweighted).
-template <typename T, int VPW, int NEM, int M, bool RESID, bool EDGEX>
-__global__ __launch_bounds__(256, (fwd_waves<T, NEM, M, false>())) void k_fwd_lt(
-    DevPlan P, const double2* __restrict__ lt, T* __restrict__ y, int B, int ngx, int ngy,
-    const double* __restrict__ post, const T* __restrict__ m, double2* __restrict__ tabs, int nch,
-    double* __restrict__ rowsq) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int nwx = B * ngx;
-    int w = xcd_remap(blockIdx.x, gridDim.x, (nwx + B * ngy) * nch);
-    if (w < 0) return;
-    const int ch = w % nch;
-    w /= nch;
-    const int mode = w < nwx ? MODE_X : MODE_Y;
-    if (mode == MODE_Y) w -= nwx;
-    const int ngroups = mode == MODE_Y ? ngy : ngx;
-    const int b = w / ngroups, grp = w - b * ngroups;
-    const int nl = mode == MODE_Y ? P.W : P.H;
+// The same packed by four slices (fp32 data): one wave per line of a group, each slice's table as
+// line_table_wave forms it, stored as {C_0, C_1}, {C_2, C_3} and {S_0 .. S_3}.
+template <int M>
+__global__ __launch_bounds__(256) void k_line_tables4(DevPlan P, const float* __restrict__ srcx,
+                                                      const float* __restrict__ srcy, double2* __restrict__ lt, int B) {
     const int hx = P.nx ? P.H : 0, wy = P.ny ? P.W : 0;
-    const double2* lts = lt + ((size_t)b * (hx + wy) + (mode == MODE_Y ? hx : 0)) * ltab_n<M>();
-    fwd_block_lt<T, VPW, NEM, M, RESID, EDGEX, FWD_LT_BUFFERS>(P, lts, y + (size_t)ch * B * P.V * P.D, b, mode, grp, post,
-                                                          m, tabs, smem, ch * nl / nch, (ch + 1) * nl / nch, rowsq);
+    const int nl = hx + wy;
+    const int line = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (line >= (B + 3) / 4 * nl) return;  // whole wave
+    const int g = line / nl, l = line - g * nl;
+    const int n = l < hx ? P.W : P.H;
+    constexpr int TABN = ltab_n<M>();
+    const float* row[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const size_t b = min(4 * g + s, B - 1);
+        row[s] = l < hx ? srcx + (b * P.H + l) * P.W : srcy + (b * P.W + (l - hx)) * P.H;
+    }
+    double2* c01 = lt + (size_t)line * 3 * TABN;
+    double2* c23 = c01 + TABN;
+    float4* sl = reinterpret_cast<float4*>(c23 + TABN);
+    double carry[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+    for (int k = 0; 64 * k < n; k++) {
+        const int p = 64 * k + lane;
+        float v[4];
+        double c[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) v[s] = p < n ? row[s][p] : 0.0f;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const double x = (double)v[s], inc = wave_scan_incl(x, lane);
+            c[s] = carry[s] + (inc - x) - (double)(p + 1) * x;
+            carry[s] += readlane_d(inc, 63);
+        }
+        if (p < n) {
+            c01[p + 1] = make_double2(c[0], c[1]);
+            c23[p + 1] = make_double2(c[2], c[3]);
+            sl[p + 1] = make_float4(v[0], v[1], v[2], v[3]);
+        }
+    }
+    if (lane == 0) {
+        c01[0] = c23[0] = make_double2(0.0, 0.0);
+        c01[n + 1] = make_double2(carry[0], carry[1]);
+        c23[n + 1] = make_double2(carry[2], carry[3]);
+        sl[0] = sl[n + 1] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
 }
 
 // One launch covers both sweep axes: work items [0, B*ngx) are (b, group of
@@ -199,11 +222,16 @@ int fwd_px(const DevPlan& P) {
     return m <= 2 ? 2 : m <= 4 ? 4 : m <= 8 ? 8 : 0;
 }
 
+bool fwd_packed(const DevPlan& P, int dtype, int64_t B) {
+    const int M = fwd_px(P);
+    return dtype == DT_F32 && M >= 1 && M <= 2 && (B % 4 == 0 || B % 4 == 3 || B >= 9);
+}
+
 size_t fwd_line_table_bytes(const DevPlan& P, int B) {
     const int M = fwd_px(P);
     if (B <= 0 || M == 0 || P.nx + P.ny == 0) return 0;
     const size_t nlt = (size_t)(P.nx ? P.H : 0) + (P.ny ? P.W : 0);
-    return (size_t)B * nlt * (NT * M + 2) * sizeof(double2);
+    return ((size_t)B * nlt * (NT * M + 2) + 64) * sizeof(double2);
 }
 
 size_t fwd_lds_bytes(const DevPlan& P, bool weighted, int G) {
@@ -224,7 +252,6 @@ struct FwdArgs {
     double2* tabs;
     int nch;
     double* rowsq;
-    const double2* lt;  // line tables of launch_line_tables (unweighted), or null: each block builds its own
 };
 
 template <typename T, int VPW, int NEM, int M, bool WTD, bool RESID, bool FULL, bool EDGEX>
@@ -234,19 +261,6 @@ hipError_t fwd_launch_t(const DevPlan& P, const FwdArgs& a, hipStream_t s) {
     const long long nw = (long long)(ngx + ngy) * a.B * a.nch;
     if (nw > (1LL << 30)) return hipErrorInvalidValue;  // grid size (one block per work item)
     const int nwork = (int)nw;
-    if constexpr (!WTD) {
-        if (a.lt) {
-            const size_t lds = fwd_lt_lds<M>(G, FWD_LT_BUFFERS);
-            auto kern = k_fwd_lt<T, VPW, NEM, M, RESID, EDGEX>;
-            if (lds > 64 * 1024) {
-                hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-                if (e != hipSuccess) return e;
-            }
-            hipLaunchKernelGGL(kern, dim3(grid_for(nwork)), dim3(NT), lds, s, P, (const double2*)a.lt, (T*)a.y, a.B,
-                               ngx, ngy, a.post, (const T*)a.m, a.tabs, a.nch, a.rowsq);
-            return hipGetLastError();
-        }
-    }
     const size_t lds = fwd_lds_bytes(P, WTD, G);
     auto kern = k_fwd<T, VPW, NEM, M, WTD, RESID, FULL, EDGEX>;
     if (lds > 64 * 1024) {
@@ -324,6 +338,14 @@ hipError_t line_tables_t(const DevPlan& P, const void* srcx, const void* srcy, d
 hipError_t launch_line_tables(const DevPlan& P, int dtype, const void* srcx, const void* srcy, double2* ltab, int B,
                               hipStream_t s) {
     if (B <= 0 || P.nx + P.ny == 0) return hipSuccess;
+    if (fwd_packed(P, dtype, B)) {
+        const long long nw = (long long)((B + 3) / 4) * ((P.nx ? P.H : 0) + (P.ny ? P.W : 0));
+        if (nw > (1LL << 31) - 4) return hipErrorInvalidValue;
+        const dim3 grid((unsigned)((nw + 3) / 4));
+        auto kern = fwd_px(P) == 1 ? k_line_tables4<1> : k_line_tables4<2>;
+        hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, P, (const float*)srcx, (const float*)srcy, ltab, B);
+        return hipGetLastError();
+    }
     if (dtype == DT_F32) return line_tables_t<float>(P, srcx, srcy, ltab, B, s);
     return line_tables_t<double>(P, srcx, srcy, ltab, B, s);
 }
@@ -335,7 +357,11 @@ hipError_t launch_fwd(const DevPlan& P, int dtype, const void* srcx, const void*
     const int nch = shape.nch < 1 ? 1 : shape.nch;
     if ((P.nx && nch > P.H) || (P.ny && nch > P.W)) return hipErrorInvalidValue;
     if (weighted && fwd_w_supported(P)) return launch_fwd_w(P, dtype, srcx, srcy, y, B, post, nch, s);
-    FwdArgs a{srcx, srcy, y, B, post, nullptr, nullptr, nch, nullptr, weighted ? nullptr : ltab};
+    if (!weighted && ltab) {
+        const FwdGroupArgs g{ltab, y, B, post, nullptr, nullptr, nch, nullptr};
+        return dtype == DT_F32 ? launch_fwd_lt_f32(P, g, s) : launch_fwd_lt_f64(P, g, s);
+    }
+    FwdArgs a{srcx, srcy, y, B, post, nullptr, nullptr, nch, nullptr};
     if (dtype == DT_F32) return fwd_dispatch<float>(P, a, weighted, false, shape.G, s);
     return fwd_dispatch<double>(P, a, weighted, false, shape.G, s);
 }
@@ -344,7 +370,11 @@ hipError_t launch_fwd_resid(const DevPlan& P, int dtype, const void* srcx, const
                             double2* tabs, int B, FwdShape shape, hipStream_t s, double* rowsq, const double2* ltab) {
     if (B <= 0 || P.nx + P.ny == 0) return hipSuccess;
     if ((P.nx && P.W > NT * 8) || (P.ny && P.H > NT * 8) || P.D > 2046) return hipErrorInvalidValue;
-    FwdArgs a{srcx, srcy, y, B, P.post_prj, m, tabs, 1, rowsq, ltab};
+    if (ltab) {
+        const FwdGroupArgs g{ltab, y, B, P.post_prj, m, tabs, 1, rowsq};
+        return dtype == DT_F32 ? launch_fwd_lt_f32(P, g, s) : launch_fwd_lt_f64(P, g, s);
+    }
+    FwdArgs a{srcx, srcy, y, B, P.post_prj, m, tabs, 1, rowsq};
     if (dtype == DT_F32) return fwd_dispatch<float>(P, a, false, true, shape.G, s);
     return fwd_dispatch<double>(P, a, false, true, shape.G, s);
 }

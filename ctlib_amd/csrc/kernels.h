@@ -46,6 +46,17 @@ struct AdjShape {
     int NS, SL, PH, L;
     int nch;
 };
+// line->bin launch over prebuilt line tables (dd_fwd_group.h); tabs not null: also the residual tables
+struct FwdGroupArgs {
+    const double2* lt;
+    void* y;
+    int B;
+    const double* post;
+    const void* m;
+    double2* tabs;
+    int nch;
+    double* rowsq;
+};
 struct AdjArgs {
     const double2* tabs;
     void* outX;
@@ -70,15 +81,25 @@ hipError_t launch_fwd(const DevPlan& P, int dtype, const void* srcx, const void*
                       const double2* ltab = nullptr);
 // Cumulative table of every image line of both axes (one wave per line) into ltab, of
 // fwd_line_table_bytes(P, B): per slice the X-axis lines (rows of srcx) then the Y-axis lines
-// (rows of srcy), 256*M + 2 entries {C_j, S_j} per line, M = fwd_px(P).
+// (rows of srcy), 256*M + 2 entries {C_j, S_j} per line, M = fwd_px(P).  fwd_packed: per group of four
+// slices (the last slice repeated), per line the entries {C_j of slices 0, 1}, then {C_j of 2, 3}, then
+// {S_j of 0 .. 3} in fp32.
 hipError_t launch_line_tables(const DevPlan& P, int dtype, const void* srcx, const void* srcy, double2* ltab, int B,
                               hipStream_t s);
+hipError_t launch_fwd_lt_f32(const DevPlan& P, const FwdGroupArgs& a, hipStream_t s);
+hipError_t launch_fwd_lt_f64(const DevPlan& P, const FwdGroupArgs& a, hipStream_t s);
 // out[i] = sum_k parts[k*count + i], k < nch (out may equal parts)
 hipError_t launch_sum_parts(void* out, const void* parts, int dtype, int nch, size_t count, hipStream_t s);
 size_t fwd_lds_bytes(const DevPlan& P, bool weighted, int G);
 // Pixels per thread M of the line -> bin launch (lines of at most 256*M pixels; 0: too long).
 int fwd_px(const DevPlan& P);
-// Bytes of the prebuilt line tables of a batch of B: B * (lines of both axes) * (256*M + 2) * 16.
+// Whether the line tables of a batch are packed by four slices (dd_fwd_group.h): fp32 data, lines up to
+// 512 pixels (a CU holds the buffers of only one block of packed longer ones: fan-ED 1024^2 B=4 2.15 ms
+// against 2.07 in pairs), and few enough slots of the last group empty that it pays - a packed group of four costs
+// 1.6 pairs (they also need no more memory then: 48 bytes an entry and group against 16 and slice).
+bool fwd_packed(const DevPlan& P, int dtype, int64_t B);
+// Bytes of the prebuilt line tables of a batch of B (an upper bound where they are packed): (B * (lines of both axes) * (256*M + 2) + 64) * 16,
+// the last 64 entries because the line -> bin kernel copies whole chunks of 64.
 size_t fwd_line_table_bytes(const DevPlan& P, int B);
 
 // projection fused with the residual bin tables of projection_t: writes y = A x (y may be null)
