@@ -675,125 +675,6 @@ __device__ __forceinline__ void fwd_block_lt(const DevPlan& P, const double2* __
     fwd_store<T, VPW, NEM, RESID, EDGEX>(P, S, vw, grp, b, mode, lane, wave, y, post, m, tabs, Sx, rowsq);
 }
 
-// Entries of a wave-private line table sit at j + j/8 (one 16-byte pad every 8):
-// lane L writes entries 8L+1 .. 8L+8, and with the pad consecutive lanes land
-// 9 entries apart, so each ds_write_b128 of 16 lanes covers all 64 banks.
-__host__ __device__ inline int wtab_slots(int n) { return n + 2 + (n + 2) / 8 + 1; }
-__device__ __forceinline__ int wtab_slot(int j) { return j + (j >> 3); }
-
-// LDS bytes of one fwd_block_w: one wave-private table per wave.
-__host__ __device__ inline size_t fwd_w_block_lds(int nmax) { return (size_t)4 * wtab_slots(nmax) * 16; }
-
-// Weighted line -> bin work item (backprojection_t and its exact adjoint form)
-// for lines of at most 64*PPL pixels: G = 4 views per block, one per wave, and
-// each wave builds the weighted cumulative table of its own view for every line
-// by itself: lane L owns pixels L*PPL .. L*PPL+PPL-1 (one serial sum and one
-// wave scan per line) and writes them into its wave's private table, so no
-// barrier is needed anywhere.  The line's pixels and the view's LineCoef words
-// are loaded one line ahead into registers.  FULL: every line has exactly
-// 64*PPL pixels, so no lane needs a bounds predicate.  The pixel weight
-// 1/(s ((w0 + w1 p)^2 + w2)) is formed in the data precision (fp32 data: fp32
-// arithmetic with a fp32 reciprocal, about 1e-7 relative; fp64 data: fp64
-// arithmetic with a Newton-refined reciprocal), and the weighted value is rounded to the
-// data type before the fp64 prefix sum, as in fwd_block with WEIGHTED.
-// Lines [lb, le) of the axis contribute (le < 0: all), as in fwd_block.
-template <typename T, int NEM, int PPL, bool FULL>
-__device__ __forceinline__ void fwd_block_w(const DevPlan& P, const T* __restrict__ src, T* __restrict__ y, int b,
-                                            int mode, int grp, const double* __restrict__ post,
-                                            unsigned char* __restrict__ smem, int lb = 0, int le = -1) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int* vlist = mode == MODE_Y ? P.yviews : P.xviews;
-    const int nv = mode == MODE_Y ? P.ny : P.nx;
-    const int nlines = mode == MODE_Y ? P.W : P.H;
-    const int n = FULL ? 64 * PPL : (mode == MODE_Y ? P.H : P.W);
-    const int D = P.D;
-
-    int vw[1];
-    {
-        const int idx = grp * 4 + wave;
-        vw[0] = vlist[idx < nv ? idx : nv - 1];
-    }
-    double e[1][NEM], S[1][NEM];
-#pragma unroll
-    for (int i = 0; i < NEM; i++) {
-        const int k = lane + 64 * i;
-        e[0][i] = P.edges[(size_t)vw[0] * (D + 1) + (k <= D ? k : D)];
-        S[0][i] = 0.0;
-    }
-
-    double2* tb = reinterpret_cast<double2*>(smem) + (size_t)wave * wtab_slots(n);
-    const T* base = src + (size_t)b * nlines * n;
-    const int p0 = lane * PPL;
-    const int hi = n + 1;
-    // LineCoef word `lane` (lanes 0..7) of this wave's view, one line ahead
-    const double* crow = reinterpret_cast<const double*>(P.lines + (size_t)vw[0] * P.max_lines) + (lane & 7);
-    // fp32 data: the line's pre-scaled weight coefficients {., c w1, c w0, c^2 w2} (uniform)
-    const float4* wrow = P.adj_wk + (size_t)vw[0] * P.max_lines;
-    auto load_line = [&](int l, T (&xv)[PPL], double& cw, float4& wk) {
-        const T* row = base + (size_t)l * n;
-#pragma unroll
-        for (int k = 0; k < PPL; k++) xv[k] = (FULL || p0 + k < n) ? row[p0 + k] : T(0);
-        cw = crow[(size_t)l * LC_WORDS];
-        if (sizeof(T) == 4) wk = wrow[l];
-    };
-    const int lend = le < 0 ? nlines : le;
-    T xv[PPL];
-    double cw = 0.0;
-    float4 wk = make_float4(0.f, 0.f, 0.f, 1.f);
-#pragma unroll
-    for (int k = 0; k < PPL; k++) xv[k] = T(0);
-    if (lb < lend) load_line(lb, xv, cw, wk);
-
-    for (int l = lb; l < lend; l++) {
-        const double s = readlane_d(cw, LC_S), A = readlane_d(cw, LC_A), Bc = readlane_d(cw, LC_B);
-        const double w0 = readlane_d(cw, LC_W0), w1 = readlane_d(cw, LC_W1);
-        const double w2 = readlane_d(cw, LC_W2), is = readlane_d(cw, LC_INVS);
-        double val[PPL];
-        if constexpr (sizeof(T) == 4) {
-            // weight (1/s) / ((w0 + w1 p)^2 + w2) = 1 / (u^2 + c^2 w2), u = k c w1 + (p0 c w1 + c w0)
-            const float u0 = __builtin_fmaf(wk.y, (float)p0, wk.z);
-#pragma unroll
-            for (int k = 0; k < PPL; k++) {
-                const float u = k == 0 ? u0 : __builtin_fmaf((float)k, wk.y, u0);
-                const float v = (float)xv[k] * __builtin_amdgcn_rcpf(__builtin_fmaf(u, u, wk.w));
-                val[k] = (FULL || p0 + k < n) ? (double)v : 0.0;
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < PPL; k++) {
-                const double u = __builtin_fma(w1, (double)(p0 + k), w0);
-                const double d = __builtin_fma(u, u, w2);
-                const double v = (double)xv[k] * (is * rcp_refined(d));
-                val[k] = (FULL || p0 + k < n) ? v : 0.0;
-            }
-        }
-        double run = 0.0;
-#pragma unroll
-        for (int k = 0; k < PPL; k++) run += val[k];
-        if (l + 1 < lend) load_line(l + 1, xv, cw, wk);
-        // Table of this line: the wave's reads of the previous line's table were
-        // consumed above (in-order LDS within a wave), so it can be overwritten.
-        const double inc = wave_scan_incl(run, lane);
-        double pref = inc - run;
-#pragma unroll
-        for (int k = 0; k < PPL; k++) {
-            const int p = p0 + k;
-            if (FULL || p < n) tb[wtab_slot(p + 1)] = make_double2(__builtin_fma(-(double)(p + 1), val[k], pref), val[k]);
-            pref += val[k];
-        }
-        if (lane == 0) tb[0] = make_double2(0.0, 0.0);
-        if (lane == 63) tb[wtab_slot(n + 1)] = make_double2(inc, 0.0);
-#pragma unroll
-        for (int i = 0; i < NEM; i++) {
-            const double tau = __builtin_fma(A, e[0][i], Bc);
-            const double2 ent = tb[wtab_slot(table_index_d(tau, hi))];
-            S[0][i] = __builtin_fma(s, __builtin_fma(tau, ent.y, ent.x), S[0][i]);
-        }
-    }
-    fwd_store<T, 1, NEM, false>(P, S, vw, grp, b, mode, lane, wave, y, post, nullptr, nullptr);
-}
-
 // ---------------------------------------------------------------------------
 // Bin -> pixel (projection_t / backprojection)
 // ---------------------------------------------------------------------------

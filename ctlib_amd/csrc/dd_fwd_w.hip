@@ -1,9 +1,9 @@
 // Stand-alone launch of the weighted line -> bin kernel with wave-private line
-// tables (fwd_block_w in dd_device.h): backprojection_t and the exact adjoint of
+// tables (fwd_group_w in dd_fwd_w_group.h): backprojection_t and the exact adjoint of
 // backprojection, for lines of at most 1024 pixels.
 #include <hip/hip_runtime.h>
 
-#include "dd_device.h"
+#include "dd_fwd_w_group.h"
 #include "kernels.h"
 
 namespace ctlib {
@@ -12,30 +12,30 @@ using namespace dd;
 
 namespace {
 
-// Work items [0, B*ngx) are (b, group of 4 X-axis views) reading image rows from
+// Work items [0, ngrp*ngx) are (slice group, 4 X-axis views) reading image rows from
 // `srcx`; the rest are Y-axis groups reading the bottom-to-top column copy.
 // fp32 variants for 512-pixel lines are held to 128 VGPRs: four waves per
 // SIMD, as many as the LDS of four 512-pixel tables per block allows.
 template <typename T, int NEM, int PPL, bool FULL>
-constexpr int fwd_w_waves() { return sizeof(T) == 4 && FULL && PPL == 8 && NEM <= 12 ? 4 : 1; }
+constexpr int fwd_w_waves() { return sizeof(T) == 4 && FULL && PPL == 8 && NEM <= 14 ? 4 : 1; }
 
-template <typename T, int NEM, int PPL, bool FULL>
+template <typename T, int NS, int NEM, int PPL, bool FULL>
 __global__ __launch_bounds__(256, (fwd_w_waves<T, NEM, PPL, FULL>())) void k_fwd_w(DevPlan P, const T* __restrict__ srcx, const T* __restrict__ srcy,
-                                               T* __restrict__ y, int B, int ngx, int ngy,
+                                               T* __restrict__ y, int B, int ngrp, int ngx, int ngy,
                                                const double* __restrict__ post, int nch) {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int nwx = B * ngx;
-    int w = xcd_remap(blockIdx.x, gridDim.x, (nwx + B * ngy) * nch);
+    const int nwx = ngrp * ngx;
+    int w = xcd_remap(blockIdx.x, gridDim.x, (nwx + ngrp * ngy) * nch);
     if (w < 0) return;
     const int ch = w % nch;
     w /= nch;
     const int mode = w < nwx ? MODE_X : MODE_Y;
     if (mode == MODE_Y) w -= nwx;
     const int ngroups = mode == MODE_Y ? ngy : ngx;
-    const int b = w / ngroups, grp = w - b * ngroups;
+    const int sg = w / ngroups, grp = w - sg * ngroups;
     const int nl = mode == MODE_Y ? P.W : P.H;
-    fwd_block_w<T, NEM, PPL, FULL>(P, mode == MODE_Y ? srcy : srcx, y + (size_t)ch * B * P.V * P.D, b, mode, grp,
-                                   post, smem, ch * nl / nch, (ch + 1) * nl / nch);
+    fwd_group_w<T, NS, NEM, PPL, FULL>(P, mode == MODE_Y ? srcy : srcx, y + (size_t)ch * B * P.V * P.D, sg * NS, B, mode,
+                                       grp, post, smem, ch * nl / nch, (ch + 1) * nl / nch);
 }
 
 int line_max(const DevPlan& P) {
@@ -53,20 +53,20 @@ struct Args {
     int nch;
 };
 
-template <typename T, int NEM, int PPL, bool FULL>
+template <typename T, int NS, int NEM, int PPL, bool FULL>
 hipError_t launch_t(const DevPlan& P, const Args& a, hipStream_t s) {
-    const int ngx = (P.nx + 3) / 4, ngy = (P.ny + 3) / 4;
-    const long long nw = (long long)(ngx + ngy) * a.B * a.nch;
+    const int ngx = (P.nx + 3) / 4, ngy = (P.ny + 3) / 4, ngrp = (a.B + NS - 1) / NS;
+    const long long nw = (long long)(ngx + ngy) * ngrp * a.nch;
     if (nw > (1LL << 30)) return hipErrorInvalidValue;  // grid size (one block per work item)
     const int nwork = (int)nw;
     const size_t lds = fwd_w_block_lds(line_max(P));
-    auto kern = k_fwd_w<T, NEM, PPL, FULL>;
+    auto kern = k_fwd_w<T, NS, NEM, PPL, FULL>;
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL(kern, dim3(grid_for(nwork)), dim3(NT), lds, s, P, (const T*)a.srcx, (const T*)a.srcy, (T*)a.y,
-                       a.B, ngx, ngy, a.post, a.nch);
+                       a.B, ngrp, ngx, ngy, a.post, a.nch);
     return hipGetLastError();
 }
 
@@ -75,8 +75,14 @@ bool all_lines(const DevPlan& P, int n) { return (P.nx == 0 || P.W == n) && (P.n
 
 template <typename T, int NEM, int PPL>
 hipError_t by_full(const DevPlan& P, const Args& a, hipStream_t s) {
-    if (all_lines(P, 64 * PPL)) return launch_t<T, NEM, PPL, true>(P, a, s);
-    return launch_t<T, NEM, PPL, false>(P, a, s);
+    // Two slices share weights and addresses where that outweighs the registers of the second: fp64 data
+    // (dearer weights), lines up to 512 pixels and 895 bins, batches of pairs (fan-ED 512^2, 736 bins, B=8:
+    // 1.59 -> 1.41 ms; fp32 1.38 -> 1.36, with fewer waves per SIMD, and 1024-pixel lines 5.5 -> 7.4).
+    if constexpr (sizeof(T) == 8 && PPL <= 8 && NEM <= 14) {
+        if (a.B % 2 == 0 || a.B >= 9)
+            return all_lines(P, 64 * PPL) ? launch_t<T, 2, NEM, PPL, true>(P, a, s) : launch_t<T, 2, NEM, PPL, false>(P, a, s);
+    }
+    return all_lines(P, 64 * PPL) ? launch_t<T, 1, NEM, PPL, true>(P, a, s) : launch_t<T, 1, NEM, PPL, false>(P, a, s);
 }
 
 // Pixels per lane: 64 * PPL >= n.
