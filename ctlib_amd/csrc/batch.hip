@@ -25,7 +25,8 @@
 #include <vector>
 
 #include "../../include/ctlib_abi.h"
-#include "dd_device.h"
+#include "dd_adj_group.h"
+#include "dd_fwd_group.h"
 #include "kernels.h"
 
 namespace ctlib {
@@ -38,6 +39,7 @@ enum { IT_T = 0, IT_L = 1, IT_F = 2, IT_A = 3, IT_C = 4, NPHASE = 5 };
 constexpr int BAND = 64;   // image rows per T / C item
 constexpr int BG = 4;      // views per F item
 constexpr int LL = 16;     // image lines per L item (4 per wave)
+constexpr int BL = 8;      // image lines per A item (2 per wave)
 
 struct SliceDev {
     DevPlan P;
@@ -50,7 +52,7 @@ struct SliceDev {
     void* yt;
     double2* lt;  // line tables: X-axis lines then Y-axis lines, ltab_n<M>() entries each
     int fcls;   // forward variant (edge-slot class, see run_fwd)
-    int acls;   // adjoint variant: line class * 4 + GEO (GEO_EAP for fan-EA with the polynomial atan)
+    int acls;   // adjoint variant: line class (run_adj) * 4 + GEO (GEO_EAP for fan-EA with the polynomial atan)
     int ngx, ngy, ntx, nty, nband;
     int nlx, nly;  // L items of each axis
     int tileL;  // image lines per adjoint item
@@ -82,59 +84,63 @@ __device__ __forceinline__ void run_lines(const SliceDev& sd, int mode, int idx)
     }
 }
 
-// Forward of one F item over the slice's line tables.  Edge slots per view: 12 (D < 768), 20
-// (D < 1280) or 24 (D < 1536); 512, 1024 or 1536 bins: 8, 16 or 24 slots and the last edge packed.
-template <typename T, bool LARGE>
-__device__ __forceinline__ void run_fwd(const SliceDev& sd, int mode, int grp, unsigned char* smem) {
+// Forward of one F item over the slice's line tables: one slice's form of the stand-alone kernel.
+// Edge slots per view: 12 (D < 768), 20 (D < 1280) or 24 (D < 1536); 512, 1024 or 1536 bins: 8, 16 or
+// 24 slots and the last edge apart.
+template <typename T, bool LARGE, int NE, bool EXTRA>
+__device__ __forceinline__ void run_fwd_ne(const SliceDev& sd, int mode, int grp, unsigned char* smem) {
     constexpr int M = batch_px<LARGE>();
-    T* y = (T*)sd.y;
-    const T* m = (const T*)sd.m;
     const DevPlan& P = sd.P;
     const double2* lt = sd.lt + (size_t)(mode == MODE_Y && P.nx ? P.H : 0) * ltab_n<M>();
+    fwd_group<T, 1, NE, M, true, EXTRA>(P, lt, 0, (T*)sd.y, 0, 1, mode, grp, 1, P.post_prj, (const T*)sd.m, sd.tabs,
+                                        smem, 0, mode == MODE_Y ? P.W : P.H, nullptr);
+}
+
+template <typename T, bool LARGE>
+__device__ __forceinline__ void run_fwd(const SliceDev& sd, int mode, int grp, unsigned char* smem) {
     switch (sd.fcls) {
-    case 0: fwd_block_lt<T, 1, 12, M, true, false, 2>(P, lt, y, 0, mode, grp, P.post_prj, m, sd.tabs, smem, 0, -1, nullptr); break;
-    case 2: fwd_block_lt<T, 1, 8, M, true, true, 2>(P, lt, y, 0, mode, grp, P.post_prj, m, sd.tabs, smem, 0, -1, nullptr); break;
-    case 3: fwd_block_lt<T, 1, 16, M, true, true, 2>(P, lt, y, 0, mode, grp, P.post_prj, m, sd.tabs, smem, 0, -1, nullptr); break;
+    case 0: run_fwd_ne<T, LARGE, 12, false>(sd, mode, grp, smem); break;
+    case 2: run_fwd_ne<T, LARGE, 8, true>(sd, mode, grp, smem); break;
+    case 3: run_fwd_ne<T, LARGE, 16, true>(sd, mode, grp, smem); break;
     case 4:
-        if constexpr (LARGE) fwd_block_lt<T, 1, 24, M, true, false, 2>(P, lt, y, 0, mode, grp, P.post_prj, m, sd.tabs, smem, 0, -1, nullptr);
+        if constexpr (LARGE) run_fwd_ne<T, LARGE, 24, false>(sd, mode, grp, smem);
         break;
     case 5:
-        if constexpr (LARGE) fwd_block_lt<T, 1, 24, M, true, true, 2>(P, lt, y, 0, mode, grp, P.post_prj, m, sd.tabs, smem, 0, -1, nullptr);
+        if constexpr (LARGE) run_fwd_ne<T, LARGE, 24, true>(sd, mode, grp, smem);
         break;
-    default: fwd_block_lt<T, 1, 20, M, true, false, 2>(P, lt, y, 0, mode, grp, P.post_prj, m, sd.tabs, smem, 0, -1, nullptr); break;
+    default: run_fwd_ne<T, LARGE, 20, false>(sd, mode, grp, smem); break;
     }
 }
 
-template <typename T, int LPW, int NPE, bool EXACT>
+// Adjoint of one A item: one slice's form of the stand-alone kernel on the batch's four waves, a tile
+// of BL lines.
+template <typename T, int SL>
 __device__ __forceinline__ void run_adj_geo(const SliceDev& sd, int mode, int tile, unsigned char* smem) {
     T* ox = (T*)sd.grad;
     T* oy = (T*)sd.yt;
+    const int nv = mode == MODE_Y ? sd.P.ny : sd.P.nx;
     switch (sd.acls & 3) {
-    case GEO_ED: adj_block<T, LPW, NPE, GEO_ED, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, smem); break;
-    case GEO_EA: adj_block<T, LPW, NPE, GEO_EA, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, smem); break;
-    case GEO_PARA:
-        adj_block<T, LPW, NPE, GEO_PARA, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, smem);
+    case GEO_ED: adj_group<T, 1, SL, false, GEO_ED, 4>(sd.P, sd.tabs, ox, oy, 0, 1, mode, tile, 1, 1.0, smem, 0, nv); break;
+    case GEO_PARA: adj_group<T, 1, SL, false, GEO_PARA, 4>(sd.P, sd.tabs, ox, oy, 0, 1, mode, tile, 1, 1.0, smem, 0, nv); break;
+    case GEO_EA: adj_group<T, 1, SL, false, GEO_EA, 4>(sd.P, sd.tabs, ox, oy, 0, 1, mode, tile, 1, 1.0, smem, 0, nv); break;
+    default:
+        // fp64 data takes the arctangent with atan either way
+        adj_group<T, 1, SL, false, sizeof(T) == 4 ? GEO_EAP : GEO_EA, 4>(sd.P, sd.tabs, ox, oy, 0, 1, mode, tile, 1, 1.0,
+                                                                         smem, 0, nv);
         break;
-    default: adj_block<T, LPW, NPE, GEO_EAP, EXACT>(sd.P, sd.tabs, ox, oy, 0, mode, tile, smem); break;
     }
 }
 
-// Line classes: 0 lines <= 256 px, 1 lines <= 512 px; all lines exactly 2: 256, 3: 512, 4: 384 px
-// (the last pixel edge evaluated packed); LARGE batches also 5: lines <= 1024 px, 6: exactly 1024 px.
+// Line classes (slots of 32 edges): 0 lines <= 256 px, 1 <= 384, 2 <= 512; LARGE batches also 3, <= 1024.
 template <typename T, bool LARGE>
 __device__ __forceinline__ void run_adj(const SliceDev& sd, int mode, int tile, unsigned char* smem) {
     switch (sd.acls >> 2) {
-    case 0: run_adj_geo<T, 8, 5, false>(sd, mode, tile, smem); break;
-    case 2: run_adj_geo<T, 8, 5, true>(sd, mode, tile, smem); break;
-    case 3: run_adj_geo<T, 4, 9, true>(sd, mode, tile, smem); break;
-    case 4: run_adj_geo<T, 4, 7, true>(sd, mode, tile, smem); break;
-    case 5:
-        if constexpr (LARGE) run_adj_geo<T, 2, 17, false>(sd, mode, tile, smem);
+    case 0: run_adj_geo<T, 8>(sd, mode, tile, smem); break;
+    case 1: run_adj_geo<T, 12>(sd, mode, tile, smem); break;
+    case 3:
+        if constexpr (LARGE) run_adj_geo<T, 32>(sd, mode, tile, smem);
         break;
-    case 6:
-        if constexpr (LARGE) run_adj_geo<T, 2, 17, true>(sd, mode, tile, smem);
-        break;
-    default: run_adj_geo<T, 4, 9, false>(sd, mode, tile, smem); break;
+    default: run_adj_geo<T, 16>(sd, mode, tile, smem); break;
     }
 }
 
@@ -159,11 +165,12 @@ __global__ void k_batch_reset(unsigned int* ctr, int n) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) ctr[i] = 0u;
 }
 
-// Register budget: 128 VGPRs (four waves per SIMD) for batches of slices within 512^2 and 1279
-// bins - 7.22 ms for the 64-slice batch against 7.66 ms at 168 (three waves) - and 168 for the
-// LARGE variant, whose 24-slot forward needs more.
+// Register budget: 168 VGPRs (three waves per SIMD) for batches of slices within 512^2 and 1279 bins,
+// 256 for the LARGE variant: within 128 the phases' loops reload spilled registers, and each reload
+// waits for the table copies under way (16 mixed slices: 2.46 ms with 4 blocks per CU against 2.88;
+// 3.28 ms with the phases' former lane order and copies, at 128).
 template <typename T, bool LARGE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LARGE ? 3 : 4))) void k_batch(const SliceDev* __restrict__ slices, const Item* __restrict__ items,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LARGE ? 2 : 3))) void k_batch(const SliceDev* __restrict__ slices, const Item* __restrict__ items,
                                                int nitems, unsigned int* __restrict__ ctr, int nslices) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int s_item;
@@ -360,18 +367,9 @@ int ctlib_batch_create(const ctlib_geom* geoms, int nslices, int device, int dty
         const int nmax = std::max(P.nx ? P.W : 0, P.ny ? P.H : 0);
         // forward class (run_fwd; 4 and 5 occur only in LARGE batches)
         sd.fcls = P.D == 512 ? 2 : P.D == 1024 ? 3 : P.D == 1536 ? 5 : ne <= 12 ? 0 : ne <= 20 ? 1 : 4;
-        const int npe = (nmax + 1 + 63) / 64;
-        // every line (rows of X views, columns of Y views) exactly n pixels
-        auto all_lines = [&](int n) { return (P.nx == 0 || P.W == n) && (P.ny == 0 || P.H == n); };
-        const int lcls = all_lines(256)    ? 2
-                         : all_lines(512)  ? 3
-                         : all_lines(384)  ? 4
-                         : all_lines(1024) ? 6
-                         : npe <= 5        ? 0
-                         : npe <= 9        ? 1
-                                           : 5;
+        const int lcls = nmax <= 256 ? 0 : nmax <= 384 ? 1 : nmax <= 512 ? 2 : 3;
         sd.acls = lcls * 4 + (P.scan_type == GEO_EA && P.ea_poly ? GEO_EAP : P.scan_type);
-        const int L = lcls == 0 || lcls == 2 ? 32 : lcls >= 5 ? 8 : 16;
+        const int L = BL;
         sd.tileL = L;
         sd.ngx = (P.nx + BG - 1) / BG;
         sd.ngy = (P.ny + BG - 1) / BG;
@@ -390,7 +388,9 @@ int ctlib_batch_create(const ctlib_geom* geoms, int nslices, int device, int dty
         off += align_up((size_t)P.H * P.W * es);                   // yt
         b->ws_off.push_back(0);  // line tables: placed once every slice's size class is known
         lines_total.push_back((size_t)(P.nx ? P.H : 0) + (P.ny ? P.W : 0));
-        b->lds = std::max(b->lds, adj_block_lds(P.D, L));
+        const int cover = lcls == 0 ? 256 : lcls == 1 ? 384 : lcls == 2 ? 512 : 1024;
+        b->lds = std::max(b->lds, dtype == CTLIB_F64 ? adjg_lds<double, 1, false>(P.D, L, cover)
+                                                     : adjg_lds<float, 1, false>(P.D, L, cover));
     }
     // line tables last (their entry count per line depends on the batch's pixels-per-thread class)
     {
@@ -399,7 +399,8 @@ int ctlib_batch_create(const ctlib_geom* geoms, int nslices, int device, int dty
             b->ws_off[4 * s + 3] = off;
             off += align_up(lines_total[s] * tabn * sizeof(double2));
         }
-        b->lds = std::max(b->lds, b->large ? fwd_lt_lds<batch_px<true>()>(BG, 2) : fwd_lt_lds<batch_px<false>()>(BG, 2));
+        b->lds = std::max(b->lds, b->large ? fwg_lds<1, batch_px<true>()>() : fwg_lds<1, batch_px<false>()>());
+        off += 64 * sizeof(double2);  // the forward copies whole chunks of 64 entries
     }
     b->lds = std::max(b->lds, (size_t)32 * 33 * 8);
     b->ws_bytes = off;

@@ -97,14 +97,15 @@ inline size_t adjg_lds(int D, int L, int cover) {
 // chunk to spare), and the next view's coefficients beside them: one wait for this wave's copies and
 // one bare barrier per view.  Nothing in the loop is read by scalar loads, which would have the wave
 // wait for all its LDS reads.
-template <typename T, int NS, int SL, bool WEIGHTED, int GEO>
+template <typename T, int NS, int SL, bool WEIGHTED, int GEO, int NW = adjg_waves<T, NS, WEIGHTED>()>
 __device__ __forceinline__ void adj_group(const DevPlan& P, const double2* __restrict__ tabs, T* __restrict__ outX,
                                           T* __restrict__ outYT, int b0, int B, int mode, int tile, int PH,
                                           double wscale, unsigned char* __restrict__ smem, int vb, int ve) {
-    constexpr int NW = adjg_waves<T, NS, WEIGHTED>();
     constexpr bool F32 = sizeof(T) == 4;
     constexpr int NA = WEIGHTED ? 2 : 1;
-    const int tid = threadIdx.x, lane = tid & 63;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // a caller's loop over work items keeps nothing derived from it in registers
+    const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int LP = NW / PH, L = 2 * LP;
     const int* vlist = mode == MODE_Y ? P.yviews : P.xviews;

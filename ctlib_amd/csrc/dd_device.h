@@ -1,7 +1,7 @@
 // Device-side building blocks of the distance-driven projector kernels
-// (gfx950).  Each operator is written as a per-work-item block function so the
-// stand-alone kernels (dd_kernels.hip) and the persistent heterogeneous batch
-// kernel (batch.hip) run the same code.
+// (gfx950).  Each operator is written as a per-work-item block function (here, in
+// dd_fwd_group.h, dd_fwd_w_group.h and dd_adj_group.h) so the stand-alone kernels
+// and the persistent heterogeneous batch kernel (batch.hip) run the same code.
 //
 // Every operator of the family (fan_ed_kernel.cu, fan_ea_kernel.cu,
 // para_kernel.cu) is, per view and per image line, the overlap-weighted
@@ -363,7 +363,7 @@ __host__ __device__ inline size_t fwd_block_lds(int nmax, int G, bool weighted, 
     return (size_t)2 * ntab * (nmax + 2) * entry_bytes + (size_t)2 * G * LC_WORDS * 8 + (size_t)2 * ntab * 4 * 8;
 }
 
-// ---- Line tables built once per (slice, line), then streamed into LDS ----
+// ---- Line tables built once per (slice, line), then streamed into LDS (dd_fwd_group.h) ----
 // Per line TABN = 256*M + 2 entries {C_j, S_j} (16 bytes, j = 0..n+1 used), the same
 // layout in global memory and in LDS, so one linear copy moves a table.
 template <int M>
@@ -538,143 +538,6 @@ __device__ __forceinline__ void fwd_block(const DevPlan& P, const T* __restrict_
     fwd_store<T, VPW, NEM, RESID, EDGEX>(P, S, vw, grp, b, mode, lane, wave, y, post, m, tabs, Sx, rowsq);
 }
 
-// LDS bytes of one fwd_block_lt: NB line-table buffers and NB LineCoef buffers.
-template <int M>
-__host__ __device__ inline size_t fwd_lt_lds(int G, int NB) {
-    return (size_t)NB * ltab_n<M>() * 16 + (size_t)NB * G * LC_WORDS * 8;
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vm_lgkm() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
-}
-
-// fwd_block over prebuilt line tables (unweighted; k_line_tables): `lt` holds the axis's
-// lines, ltab_n<M>() entries each, so a line costs no scan and one barrier, and `src` is not
-// needed.  Line l's table and the G LineCoefs of line l are copied global -> LDS by
-// global_load_lds_dwordx4 (16 bytes per lane straight into LDS, no register staging; the
-// LineCoefs by wave 0's lanes < 4G) NB - 1 lines ahead into buffer l % NB.  NB = 2 is used:
-// three buffers (two lines ahead) measured 2-4 % slower on 1024-pixel lines, where their LDS
-// lowers the blocks per CU.  Per line one wait and one barrier: each wave waits until at most
-// the copies of the lines after l are outstanding (loads complete in order), then the barrier
-// makes every wave's copies of line l visible and frees the buffer of line l - 1.  Wave w
-// issues ceil((TABN - 64 w) / 256) table copies per line (M + 1 for wave 0, M for the
-// others) and wave 0 one LineCoef copy; the waits count exactly those.
-template <typename T, int VPW, int NEM, int M, bool RESID, bool EDGEX, int NB>
-__device__ __forceinline__ void fwd_block_lt(const DevPlan& P, const double2* __restrict__ lt, T* __restrict__ y,
-                                             int b, int mode, int grp, const double* __restrict__ post,
-                                             const T* __restrict__ m, double2* __restrict__ tabs,
-                                             unsigned char* __restrict__ smem, int lb, int le,
-                                             double* __restrict__ rowsq) {
-    static_assert(NB == 2 || NB == 3, "two or three buffers");
-    constexpr int G = 4 * VPW;
-    constexpr int TABN = ltab_n<M>();
-    static_assert(4 * G <= 64, "one LineCoef copy instruction per line");
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int* vlist = mode == MODE_Y ? P.yviews : P.xviews;
-    const int nv = mode == MODE_Y ? P.ny : P.nx;
-    const int nlines = mode == MODE_Y ? P.W : P.H;
-    const int lend = le < 0 ? nlines : le;
-    const int n = mode == MODE_Y ? P.H : P.W;
-    const int D = P.D;
-
-    int vw[VPW];
-#pragma unroll
-    for (int v = 0; v < VPW; v++) {
-        const int idx = grp * G + wave * VPW + v;
-        vw[v] = vlist[idx < nv ? idx : nv - 1];
-    }
-    double e[VPW][NEM], S[VPW][NEM];
-#pragma unroll
-    for (int v = 0; v < VPW; v++) {
-#pragma unroll
-        for (int i = 0; i < NEM; i++) {
-            const int k = lane + 64 * i;
-            e[v][i] = P.edges[(size_t)vw[v] * (D + 1) + (k <= D ? k : D)];
-            S[v][i] = 0.0;
-        }
-    }
-    const int vxl = lane < VPW ? lane : 0;
-    int vx = vw[0];
-#pragma unroll
-    for (int v = 1; v < VPW; v++)
-        if (vxl == v) vx = vw[v];
-    const double ex = EDGEX ? P.edges[(size_t)vx * (D + 1) + D] : 0.0;
-    double Sx = 0.0;
-
-    LEnt<T>* tab = reinterpret_cast<LEnt<T>*>(smem);             // [NB][TABN]
-    double* cf = reinterpret_cast<double*>(tab + NB * TABN);    // [NB][G][LC_WORDS]
-    const int hi = n + 1;
-    const bool clane = wave == 0 && lane < 4 * G;
-    const char* csrc = nullptr;
-    if (clane) {
-        const int idx = grp * G + (lane >> 2);
-        csrc = reinterpret_cast<const char*>(P.lines + (size_t)vlist[idx < nv ? idx : nv - 1] * P.max_lines) +
-               16 * (lane & 3);
-    }
-    auto issue = [&](int l, int buf) {
-        const double2* srct = lt + (size_t)l * TABN;
-        LEnt<T>* dst = tab + buf * TABN;
-#pragma unroll
-        for (int r = 0; r < (TABN + NT - 1) / NT; r++) {
-            const int j0 = wave * 64 + r * NT;
-            if (j0 < TABN && j0 + lane < TABN)
-                __builtin_amdgcn_global_load_lds((const void*)(srct + j0 + lane),
-                                                 (__attribute__((address_space(3))) void*)(dst + j0), 16, 0, 0);
-        }
-        if (clane)
-            __builtin_amdgcn_global_load_lds((const void*)(csrc + (size_t)l * sizeof(LineCoef)),
-                                             (__attribute__((address_space(3))) void*)(cf + buf * G * LC_WORDS), 16,
-                                             0, 0);
-    };
-#pragma unroll
-    for (int k = 0; k < NB - 1; k++)
-        if (lb + k < lend) issue(lb + k, k);
-
-    int bcur = 0;
-    for (int l = lb; l < lend; l++) {
-        // copies of line l complete (at most those of line l + 1 outstanding when NB = 3)
-        if (NB == 3 && l + 1 < lend) {
-            if (wave == 0)
-                wait_vm_lgkm<M + 2>();
-            else
-                wait_vm_lgkm<M>();
-        } else {
-            wait_vm_lgkm<0>();
-        }
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        if (l + NB - 1 < lend) issue(l + NB - 1, bcur == 0 ? NB - 1 : bcur - 1);
-        const LEnt<T>* tb = tab + bcur * TABN;
-        const double* cfl = cf + bcur * G * LC_WORDS;
-        if (EDGEX) {
-            const int g = wave * VPW + vxl;
-            const double tau = __builtin_fma(cfl[g * LC_WORDS + LC_A], ex, cfl[g * LC_WORDS + LC_B]);
-            double c, sl;
-            lent_read(tb + table_index_d(tau, hi), c, sl);
-            Sx = __builtin_fma(cfl[g * LC_WORDS + LC_S], __builtin_fma(tau, sl, c), Sx);
-        }
-#pragma unroll
-        for (int v = 0; v < VPW; v++) {
-            const int g = wave * VPW + v;
-            const double s = cfl[g * LC_WORDS + LC_S];
-            const double A = cfl[g * LC_WORDS + LC_A];
-            const double Bc = cfl[g * LC_WORDS + LC_B];
-#pragma unroll
-            for (int i = 0; i < NEM; i++) {
-                const double tau = __builtin_fma(A, e[v][i], Bc);
-                double c, sl;
-                lent_read(tb + table_index_d(tau, hi), c, sl);
-                S[v][i] = __builtin_fma(s, __builtin_fma(tau, sl, c), S[v][i]);
-            }
-        }
-        bcur = bcur == NB - 1 ? 0 : bcur + 1;
-    }
-
-    fwd_store<T, VPW, NEM, RESID, EDGEX>(P, S, vw, grp, b, mode, lane, wave, y, post, m, tabs, Sx, rowsq);
-}
-
 // ---------------------------------------------------------------------------
 // Bin -> pixel (projection_t / backprojection)
 // ---------------------------------------------------------------------------
@@ -796,190 +659,6 @@ __device__ __forceinline__ double eval_G_lk(const double2* __restrict__ t, doubl
     }
     const double2 c = t[table_index(q, hi)];
     return __builtin_fma(pi, c.y, c.x);
-}
-
-// LDS bytes of one adj_block.
-__host__ __device__ inline size_t adj_block_lds(int D, int L) {
-    return (size_t)2 * (D + 2) * 16 + (size_t)2 * L * LC_WORDS * 8 + (size_t)2 * L * 16;
-}
-
-// One bin -> pixel work item: batch element b, sweep axis `mode`, image lines
-// [tile*L, tile*L + L) (L = 4*LPW; rows for X, columns bottom-to-top for Y)
-// over all views of that axis.  X lines are written to outX [B][H][W], Y lines
-// to outYT [B][W][H].  Per view: the next view's bin table is copied
-// global -> LDS with global_load_lds_dwordx4 (asynchronous, no register
-// staging) and the next view's LineCoefs of the tile are prefetched into one
-// register per thread while the current view is evaluated; one barrier per view.
-// EXACT: every line has exactly 64*(NPE-1) pixels, so its last pixel edge n is
-// the only edge of group NPE-1; instead of a ninth (or seventeenth) group per
-// line, lane q of the wave evaluates edge n of its line q (LPW <= 64 lanes),
-// one evaluation per view for all the wave's lines.
-// Used by the batch kernel, whose slices have a geometry each; the stand-alone launches share the
-// lookups of a batch's slices (dd_adj_group.h).
-template <typename T, int LPW, int NPE, int GEO, bool EXACT = false>
-__device__ __forceinline__ void adj_block(const DevPlan& P, const double2* __restrict__ tabs, T* __restrict__ outX,
-                                          T* __restrict__ outYT, int b, int mode, int tile,
-                                          unsigned char* __restrict__ smem) {
-    constexpr int L = 4 * LPW;
-    constexpr int NG = EXACT ? NPE - 1 : NPE;  // edge groups evaluated per line
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int* vlist = mode == MODE_Y ? P.yviews : P.xviews;
-    const int nv = mode == MODE_Y ? P.ny : P.nx;
-    const int nlines = mode == MODE_Y ? P.W : P.H;
-    const int n = mode == MODE_Y ? P.H : P.W;
-    const int D = P.D;
-    const int npe = (n + 1 + 63) / 64;  // edge groups (<= NPE)
-    const float hi = (float)(D + 1);
-    const int tabn = D + 2;
-
-    double2* stab = reinterpret_cast<double2*>(smem);          // [2][tabn]
-    double* scf = reinterpret_cast<double*>(stab + 2 * tabn);  // [2][L][LC_WORDS]
-    float4* slk = reinterpret_cast<float4*>(scf + 2 * L * LC_WORDS);  // [2][L] composed lookups (fp32 data)
-    constexpr bool LK = sizeof(T) == 4;
-
-    const double2* tb_b = tabs + (size_t)b * P.V * tabn;
-    // Asynchronous copy of view v's table into LDS buffer `buf`: wave w copies
-    // entries [64*(w + 4r), 64*(w + 4r) + 64); lanes past the end are masked off.
-    auto table_to_lds = [&](int v, int buf) {
-        const double2* src = tb_b + (size_t)v * tabn;
-        for (int j0 = wave * 64; j0 < tabn; j0 += NT) {
-            if (j0 + lane < tabn)
-                __builtin_amdgcn_global_load_lds((const void*)(src + j0 + lane),
-                                                 (__attribute__((address_space(3))) void*)(stab + buf * tabn + j0), 16,
-                                                 0, 0);
-        }
-    };
-    // LineCoef word `tid % 8` of tile line `tid / 8`, held by thread tid < L*8.
-    const bool cthread = tid < L * LC_WORDS;
-    const int cl = tile * L + tid / LC_WORDS;
-    const bool cvalid = cthread && cl < nlines;
-    auto coef_word = [&](int v) {
-        return cvalid ? reinterpret_cast<const double*>(P.lines + (size_t)v * P.max_lines + cl)[tid % LC_WORDS] : 0.0;
-    };
-    // composed lookup of tile line `tid`, held by thread tid < L (fp32 data)
-    const bool athread = LK && tid < L;
-    const int al = tile * L + tid;
-    auto lk_word = [&](int v) {
-        return athread && al < nlines ? P.adj_lk[(size_t)v * P.max_lines + al] : make_float4(0.f, 0.f, 0.f, 1.f);
-    };
-
-    // Tiles of 16 or more lines (DMA): the LineCoefs (16 bytes of line tid/4 per thread
-    // tid < 4L) and composed lookups (thread tid < L) are copied global -> LDS like the table,
-    // and each view ends with the wait for this wave's copies and a bare barrier instead of
-    // register-staged words and __syncthreads() (whose workgroup fence drains every access):
-    // projection_t 3-4 % faster at fan-ED 512^2, 1-2 % on fan-EA; 8-line tiles (lines over 512
-    // pixels) measured 1.5-2.5 % slower that way and keep the staged words.
-    constexpr bool DMA = LPW >= 4;
-    auto side_to_lds = [&](int v, int buf) {
-        if (tid < 4 * L) {
-            const int c4 = min(tile * L + (tid >> 2), nlines - 1);
-            __builtin_amdgcn_global_load_lds(
-                (const void*)(reinterpret_cast<const char*>(P.lines + (size_t)v * P.max_lines + c4) + 16 * (tid & 3)),
-                (__attribute__((address_space(3))) void*)(scf + buf * L * LC_WORDS + wave * 128), 16, 0, 0);
-        }
-        if (LK && tid < L)
-            __builtin_amdgcn_global_load_lds((const void*)(P.adj_lk + (size_t)v * P.max_lines + min(al, nlines - 1)),
-                                             (__attribute__((address_space(3))) void*)(slk + buf * L), 16, 0, 0);
-    };
-    auto view_barrier = [&]() {
-        if (DMA) {
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-        } else {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
-        }
-    };
-
-    double acc[LPW][NG];
-#pragma unroll
-    for (int q = 0; q < LPW; q++)
-#pragma unroll
-        for (int i = 0; i < NG; i++) acc[q][i] = 0.0;
-    double accx = 0.0;                          // EXACT: lane q accumulates edge n of line q
-    const int lx = (lane < LPW ? lane : 0) * 4 + wave;  // that line within the tile
-
-    table_to_lds(vlist[0], 0);
-    if (DMA) {
-        side_to_lds(vlist[0], 0);
-    } else {
-        if (cthread) scf[tid] = coef_word(vlist[0]);
-        if (athread) slk[tid] = lk_word(vlist[0]);
-    }
-    view_barrier();
-
-    for (int iv = 0; iv < nv; iv++) {
-        const int cur = iv & 1;
-        const int v = vlist[iv];
-        double cnext = 0.0;
-        float4 anext = make_float4(0.f, 0.f, 0.f, 1.f);
-        if (iv + 1 < nv) {
-            const int vn = vlist[iv + 1];
-            table_to_lds(vn, cur ^ 1);
-            if (DMA) {
-                side_to_lds(vn, cur ^ 1);
-            } else {
-                cnext = coef_word(vn);
-                if (athread) anext = lk_word(vn);
-            }
-        }
-        const double2* t = stab + cur * tabn;
-        const double* cf = scf + cur * L * LC_WORDS;
-        const float4* clk = slk + cur * L;
-        const Lookup lu = view_lookup(P, v);
-        if (EXACT) accx += eval_G<GEO, sizeof(T) == 8>(t, cf[lx * LC_WORDS + LC_A0], cf[lx * LC_WORDS + LC_S], n, lu, hi);
-#pragma unroll
-        for (int q = 0; q < LPW; q++) {
-            const int lq = q * 4 + wave;  // line within the tile
-            const int l = tile * L + lq;
-            if (l >= nlines) continue;    // wave-uniform
-            const double a = cf[lq * LC_WORDS + LC_A0], s = cf[lq * LC_WORDS + LC_S];
-            // Every slot is evaluated, also past the last pixel edge (clamped table
-            // index, never stored): no branch between the independent evaluations,
-            // so their LDS reads overlap.
-            // G at pixel edge lane + 64 i of this line, called for i = 0, 1, 2, ... in order
-            LineLk lk{};
-            if (LK) lk = line_lk(a, s, clk[lq], lane);
-            double pir = lk.pi0;  // axis coordinate of edge lane + 64 i (fp32 data)
-            auto G_at = [&](int i) {
-                if constexpr (LK) {
-                    if (i > 0) pir += lk.s64;
-                    return eval_G_lk<GEO>(t, pir, lk, i, lu, hi);
-                } else {
-                    return eval_G<GEO, true>(t, a, s, lane + 64 * i, lu, hi);
-                }
-            };
-#pragma unroll
-            for (int i = 0; i < NG; i++) acc[q][i] += G_at(i);
-        }
-        if (!DMA && iv + 1 < nv && cthread) scf[(cur ^ 1) * L * LC_WORDS + tid] = cnext;
-        if (!DMA && iv + 1 < nv && athread) slk[(cur ^ 1) * L + tid] = anext;
-        view_barrier();
-    }
-
-    // Write pixel values.
-#pragma unroll
-    for (int q = 0; q < LPW; q++) {
-        const int l = tile * L + q * 4 + wave;
-        if (l >= nlines) continue;
-        T* dst = mode == MODE_Y ? outYT + ((size_t)b * P.W + l) * P.H : outX + ((size_t)b * P.H + l) * P.W;
-#pragma unroll
-        for (int i = 0; i < NG; i++) {
-            if (i >= npe) continue;  // wave-uniform
-            const int p = lane + 64 * i;
-            double right = shfl_next_d(acc[q][i]);
-            double r0 = 0.0;
-#pragma unroll
-            for (int k = 0; k < NG; k++)
-                if (k == i + 1) r0 = readlane_d(acc[q][k], 0);
-            if (EXACT && i == NG - 1) r0 = readlane_d(accx, q);
-            if (lane == 63) right = r0;
-            const double val = right - acc[q][i];
-            if (p < n) dst[p] = (T)val;
-        }
-    }
 }
 
 }  // namespace dd

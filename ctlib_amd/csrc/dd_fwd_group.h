@@ -63,7 +63,9 @@ __device__ __forceinline__ void fwd_group(const DevPlan& P, const double2* __res
     constexpr int NW = fwg_waves<NS>(), LB = fwg_lines<NS, M>(), TABN = ltab_n<M>(), PITCH = fwg_pitch<NS, M>();
     constexpr int NR = fwg_regions<NS>(), ENT = fwg_entries<NS, M>();
     constexpr bool PACKED = NS == 4;
-    const int tid = threadIdx.x, lane = tid & 63;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // a caller's loop over work items keeps nothing derived from it in registers
+    const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int G = NW / EH, half = wave / G, vi = wave % G;
     const int* vlist = mode == MODE_Y ? P.yviews : P.xviews;
