@@ -178,7 +178,7 @@ int adj_chunks(const ctlib_plan* p, const Tuning& T, int64_t B, bool weighted, c
     if (T.adj_nch > 0) return T.adj_nch < vmin ? T.adj_nch : vmin;
     if (weighted) {
         const int vmax = P.nx > P.ny ? P.nx : P.ny;
-        const int64_t blocks = adj_items(P, sh, B), at_once = adj_resident(sh);
+        const int64_t blocks = adj_items(P, sh, B), at_once = sh.resident;
         int best = 1;
         double least = 0;
         for (int k = 1; k <= 12 && (k == 1 || k <= vmin / 16); k++) {
@@ -377,9 +377,9 @@ int check_ws(size_t need, const void* ws, size_t ws_bytes, const char* what) {
 }
 
 hipError_t run_line_tables(const DevPlan& P, int dtype, const void* srcx, const void* srcy, double2* lt, int B,
-                           hipStream_t s) {
+                           int nch, hipStream_t s) {
     KernelTimer t(K_AUX, 0, 0, s);
-    return launch_line_tables(P, dtype, srcx, srcy, lt, B, s);
+    return launch_line_tables(P, dtype, srcx, srcy, lt, B, nch, s);
 }
 
 // Sinogram-output ops: projection and backprojection_t.
@@ -396,7 +396,7 @@ hipError_t run_to_sino(const ctlib_plan* p, int dtype, const void* in, void* out
     }
     void* dst = L.fnch > 1 ? ws + L.sp : out;
     double2* lt = weighted ? nullptr : L.line_tables(ws);
-    if (lt) e = run_line_tables(P, dtype, in, yl, lt, B, s);
+    if (lt) e = run_line_tables(P, dtype, in, yl, lt, B, L.fnch, s);
     if (e != hipSuccess) return e;
     {
         KernelTimer t(K_FWD, sweep_bytes(P, B, dtype), 0, s);
@@ -902,7 +902,7 @@ int ctlib_run_residual_loss(const ctlib_plan* p, int dtype, const void* x, const
         e = launch_to_ylines(x, yl, dt, B, P.H, P.W, s);
     }
     double2* lt = la.line_tables(w);
-    if (e == hipSuccess && lt) e = run_line_tables(P, dt, x, P.ny ? yl : nullptr, lt, B, s);
+    if (e == hipSuccess && lt) e = run_line_tables(P, dt, x, P.ny ? yl : nullptr, lt, B, la.fnch, s);
     if (e == hipSuccess && la.fnch > 1) {
         // Batch too small to fill the chip unsplit: the forward is split into line chunks, and
         // one pass sums the partial sinograms (FP64, chunk order), writes y if wanted and forms the

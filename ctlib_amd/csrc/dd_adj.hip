@@ -219,14 +219,19 @@ template <typename T, int NS, bool WEIGHTED>
 bool shape_for(const DevPlan& P, AdjShape* sh) {
     const int n = P.ny && P.H > (P.nx ? P.W : 0) ? P.H : P.W;
     const int most = adjg_most<T, NS, WEIGHTED>(P.scan_type == GEO_EA), waves = adjg_waves<T, NS, WEIGHTED>();
+    // one slice, weighted: 8 slots (four waves per SIMD) where that leaves tiles of 8 lines
+    const int limit = NS == 1 && WEIGHTED && n <= 512 ? 8 : most;
     sh->NS = NS;
     sh->PH = 1;
-    while (32 * most * sh->PH < n) sh->PH *= 2;
+    while (32 * limit * sh->PH < n) sh->PH *= 2;
     if (sh->PH > waves) return false;
     sh->SL = (n + 32 * sh->PH - 1) / (32 * sh->PH);
     if (sh->SL < 4) sh->SL = 4;
     while (!adjg_has_slots(most, sh->SL)) sh->SL++;
     sh->L = 2 * (waves / sh->PH);
+    // 256 CUs; a block of several slices fills a CU's registers and most of its LDS, and so does a
+    // weighted one of one slice past 128 registers
+    sh->resident = NS > 1 || (WEIGHTED && (sizeof(T) == 8 || sh->SL > 8)) ? 256 : 512;
     sh->nch = 1;
     return true;
 }
@@ -235,8 +240,11 @@ template <typename T, bool WEIGHTED>
 AdjShape shape_of(const DevPlan& P, int64_t B) {
     // Four slices share one lookup from batch 3 on (a block of four costs less than two of two even
     // with a slice repeated), if four double-buffered tables fit the LDS (1022 bins); else two.
+    // Weighted, lines over 512 pixels: four slices' slots leave tiles of 4 lines and less, for which the
+    // tables come in too often (fan-ED 640^2, 500 views, B=5: 0.91 ms against 0.79 unshared).
     AdjShape sh{};
-    if (B >= 3 && P.D <= adjg_max_bins<4>() && shape_for<T, 4, WEIGHTED>(P, &sh)) return sh;
+    const int n = P.ny && P.H > (P.nx ? P.W : 0) ? P.H : P.W;
+    if (B >= 3 && P.D <= adjg_max_bins<4>() && !(WEIGHTED && n > 512) && shape_for<T, 4, WEIGHTED>(P, &sh)) return sh;
     if (B >= 2 && shape_for<T, 2, WEIGHTED>(P, &sh)) return sh;
     shape_for<T, 1, WEIGHTED>(P, &sh);
     return sh;
@@ -252,9 +260,6 @@ AdjShape adj_shape(const DevPlan& P, int dtype, bool weighted, int64_t B) {
 int64_t adj_items(const DevPlan& P, const AdjShape& sh, int64_t B) {
     return (B + sh.NS - 1) / sh.NS * ((P.nx ? (P.H + sh.L - 1) / sh.L : 0) + (P.ny ? (P.W + sh.L - 1) / sh.L : 0));
 }
-
-// 256 CUs; one block of several slices fills a CU's registers and most of its LDS.
-int adj_resident(const AdjShape& sh) { return sh.NS == 1 ? 512 : 256; }
 
 int adj_tile_lines(const DevPlan& P) {
     int n = P.nx ? P.W : 0;

@@ -39,15 +39,16 @@ template <typename T, int NS, bool WEIGHTED>
 __host__ __device__ constexpr int adjg_waves() { return NS > 1 && sizeof(T) == 4 && !WEIGHTED ? 16 : 8; }
 template <typename T, int NS, bool WEIGHTED>
 __host__ __device__ constexpr int adjg_most(bool arctan) {
-    if (NS == 1) return WEIGHTED ? 8 : 16;
+    if (NS == 1) return 16;
     if (sizeof(T) == 4) return 32 / NS;
-    return (WEIGHTED ? 16 : arctan ? 40 : 64) / NS;
+    if (WEIGHTED) return NS == 4 ? 4 : arctan ? 8 : 10;
+    return (arctan ? 40 : 64) / NS;
 }
 // Slots with a kernel of their own: from half of the most on (fewer slots per wave: more waves along
-// the line instead), even ones in steps of an eighth, and 4.
+// the line instead), even ones in steps of an eighth, and 4 and 6.
 __host__ __device__ constexpr int adjg_slot_step(int most) { return most >= 32 ? 4 : 2; }
 __host__ __device__ constexpr bool adjg_has_slots(int most, int SL) {
-    return SL <= most && ((SL >= most / 2 && SL % adjg_slot_step(most) == 0) || SL == 4);
+    return SL <= most && ((SL >= most / 2 && SL % adjg_slot_step(most) == 0) || SL == 4 || SL == 6);
 }
 // The distance of the slices' tables in LDS (entries), fixed for NS > 1, which makes the slice an
 // immediate offset of the read.

@@ -29,17 +29,19 @@ namespace dd {
 template <int NS>
 __host__ __device__ constexpr int fwg_waves() { return NS == 1 ? 4 : 8; }
 template <int NS, int M>
-__host__ __device__ constexpr int fwg_lines() { return M == 1 ? (NS == 4 ? 2 : 4) : M == 2 && NS == 2 ? 2 : 1; }
-// Regions that a step's tables come from (a slice's each, or the group's packed ones), entries of 16
-// bytes of one line in a region, and a region's entries in LDS: whole chunks of 64, as they are copied.
+__host__ __device__ constexpr int fwg_lines() { return M == 1 ? (NS == 1 ? 4 : 2) : M == 2 && NS == 2 ? 2 : 1; }
+// A step's tables are rows of n + 2 entries of 16 bytes (of ltab_n<M>() in memory and LDS): per line and
+// slice one, per line of a packed group three.  A row is copied in chunks of 64, the last masked: rows
+// of whole chunks in LDS leave 256-pixel lines three blocks a CU where four fit (fan-ED 200^2, 500 views,
+// B=3: 68 us).
 template <int NS>
-__host__ __device__ constexpr int fwg_regions() { return NS == 2 ? 2 : 1; }
+__host__ __device__ constexpr int fwg_line_rows() { return NS == 4 ? 3 : NS; }
 template <int NS, int M>
-__host__ __device__ constexpr int fwg_entries() { return (NS == 4 ? 3 : 1) * ltab_n<M>(); }
+__host__ __device__ constexpr int fwg_rows() { return fwg_lines<NS, M>() * fwg_line_rows<NS>(); }
+template <int M>
+__host__ __device__ constexpr int fwg_pitch() { return ltab_n<M>(); }
 template <int NS, int M>
-__host__ __device__ constexpr int fwg_pitch() { return (fwg_lines<NS, M>() * fwg_entries<NS, M>() + 63) / 64 * 64; }
-template <int NS, int M>
-inline size_t fwg_lds() { return (size_t)2 * fwg_regions<NS>() * fwg_pitch<NS, M>() * 16; }
+inline size_t fwg_lds() { return (size_t)2 * fwg_rows<NS, M>() * fwg_pitch<M>() * 16; }
 // Slots of 64 edges a wave can have (NS sums and the edge per slot) in 128 registers; 168 from 17 on.
 template <int NS>
 __host__ __device__ constexpr int fwg_most() { return NS == 4 ? 7 : NS == 2 ? 12 : 24; }
@@ -60,8 +62,8 @@ __device__ __forceinline__ void fwd_group(const DevPlan& P, const double2* __res
                                           const double* __restrict__ post, const T* __restrict__ m,
                                           double2* __restrict__ tabs, unsigned char* __restrict__ smem, int lb, int le,
                                           double* __restrict__ rowsq) {
-    constexpr int NW = fwg_waves<NS>(), LB = fwg_lines<NS, M>(), TABN = ltab_n<M>(), PITCH = fwg_pitch<NS, M>();
-    constexpr int NR = fwg_regions<NS>(), ENT = fwg_entries<NS, M>();
+    constexpr int NW = fwg_waves<NS>(), LB = fwg_lines<NS, M>(), TABN = ltab_n<M>(), PITCH = fwg_pitch<M>();
+    constexpr int LROWS = fwg_line_rows<NS>(), ROWS = fwg_rows<NS, M>();
     constexpr bool PACKED = NS == 4;
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));  // a caller's loop over work items keeps nothing derived from it in registers
@@ -91,16 +93,23 @@ __device__ __forceinline__ void fwd_group(const DevPlan& P, const double2* __res
     for (int s = 0; s < NS; s++) Sx[s] = 0.0;
 
     const unsigned lds0 = lds_address(smem);
-    const char* tsrc = scalar_ptr(reinterpret_cast<const char*>(lt + (size_t)min(wave % NR, B - 1 - b0) * stride + (wave / NR) * 64));
+    // row r of a line: packed, row r of the line's three; else the line's table of slice b0 + r
+    const char* tsrc = reinterpret_cast<const char*>(lt);
+    const size_t row_step = 16 * (PACKED ? (size_t)TABN : B - 1 > b0 ? stride : 0);
     auto issue = [&](int l, int buf) {
-        const char* src = tsrc + (size_t)l * ENT * 16;
-        const unsigned dst = lds0 + 16 * ((buf * NR + wave % NR) * PITCH + (wave / NR) * 64);
-        const int nent = min(LB, le - l) * ENT;
-        constexpr int STEP = 64 * (NW / NR);
 #pragma unroll
-        for (int r = 0; r < (PITCH + STEP - 1) / STEP; r++) {
-            if ((wave / NR) * 64 + r * STEP >= nent) break;
-            copy_to_lds16(src + 16 * r * STEP, 16 * lane, dst + 16 * r * STEP);
+        for (int r = 0; r < ROWS; r++) {
+            const int ln = r / LROWS;
+            if (ln && l + ln >= le) break;
+            const char* src = tsrc + (size_t)(l + ln) * ((PACKED ? 3 : 1) * TABN * 16) + (r % LROWS) * row_step;
+            const unsigned dst = lds0 + 16 * (buf * ROWS + r) * PITCH;
+            // chunks of 64 entries, the first at a wave of the row's own, so that every wave has its share
+            const int first = (wave + 3 * r) % NW;
+#pragma unroll
+            for (int c = 0; c < (PITCH + 63) / 64; c += NW) {
+                if ((c + first) * 64 >= n + 2) break;
+                if (lane < n + 2 - 64 * (c + first)) copy_to_lds16(scalar_ptr(src + 1024 * (c + first)), 16 * lane, dst + 1024 * (c + first));
+            }
         }
     };
 
@@ -123,7 +132,7 @@ __device__ __forceinline__ void fwd_group(const DevPlan& P, const double2* __res
     for (int l = lb; l < le; l++) {
         const int q = (l - lb) % LB, buf = (l - lb) / LB & 1;  // line q of buffer buf
         const double sc = ns, A = nab.x, Bc = nab.y;
-        const char* t0 = reinterpret_cast<const char*>(smem) + ((size_t)buf * NR * PITCH + q * ENT) * 16;
+        const char* t0 = reinterpret_cast<const char*>(smem) + (size_t)(buf * ROWS + q * LROWS) * PITCH * 16;
         // the reads of AHEAD slots are under way while one is used
         constexpr int AHEAD = NS == 1 ? 3 : NS == 4 || (EXTRA && NE > 8) ? 1 : 2;
         double tau[AHEAD + 1];
@@ -141,8 +150,8 @@ __device__ __forceinline__ void fwd_group(const DevPlan& P, const double2* __res
             Entries t;
             if constexpr (PACKED) {
                 t.e[0] = *reinterpret_cast<const double2*>(a);
-                t.e[1] = *reinterpret_cast<const double2*>(a + TABN * 16);
-                t.s = *reinterpret_cast<const float4*>(a + 2 * TABN * 16);
+                t.e[1] = *reinterpret_cast<const double2*>(a + PITCH * 16);
+                t.s = *reinterpret_cast<const float4*>(a + 2 * PITCH * 16);
             } else {
 #pragma unroll
                 for (int s = 0; s < NS; s++) t.e[s] = *reinterpret_cast<const double2*>(a + (size_t)s * PITCH * 16);
@@ -300,9 +309,9 @@ __global__ __launch_bounds__((64 * dd::fwg_waves<NS>()), (dd::fwg_waves_per_simd
     const int sg = w / ngroups, grp = w - sg * ngroups;
     const int nl = mode == MODE_Y ? P.W : P.H;
     const int hx = P.nx ? P.H : 0, wy = P.ny ? P.W : 0;
-    const size_t stride = (size_t)(hx + wy) * dd::fwg_entries<NS, M>();  // of a slice, or of a packed group
+    const size_t stride = (size_t)(hx + wy) * ((NS == 4 ? 3 : 1) * dd::ltab_n<M>());  // of a slice, or of a packed group
     const int b0 = sg * NS;
-    const double2* lts = lt + (NS == 4 ? sg : b0) * stride + (size_t)(mode == MODE_Y ? hx : 0) * dd::fwg_entries<NS, M>();
+    const double2* lts = lt + (NS == 4 ? sg : b0) * stride + (size_t)(mode == MODE_Y ? hx : 0) * ((NS == 4 ? 3 : 1) * dd::ltab_n<M>());
     T* yc = y ? y + (size_t)ch * B * P.V * P.D : nullptr;
     dd::fwd_group<T, NS, NE, M, RESID, EXTRA>(P, lts, stride, yc, b0, B, mode, grp, EH, post, m, tabs, smem, ch * nl / nch,
                                        (ch + 1) * nl / nch, rowsq);
@@ -341,8 +350,8 @@ hipError_t fwg_edges(const DevPlan& P, const FwdGroupArgs& a, int per, int EH, h
 
 template <typename T, int NS, int M>
 hipError_t fwg_detector(const DevPlan& P, const FwdGroupArgs& a, hipStream_t s) {
-    const bool whole = P.D == 512 || P.D == 1024 || P.D == 1536;
-    const int ne = whole ? P.D / 64 : (P.D + 1 + 63) / 64;
+    const bool whole = whole_slots(P);
+    const int ne = edge_slots(P);
     int EH = 1;
     while ((ne + EH - 1) / EH > dd::fwg_most<NS>()) EH *= 2;
     if (EH > dd::fwg_waves<NS>()) return hipErrorInvalidValue;
@@ -354,14 +363,18 @@ hipError_t fwg_detector(const DevPlan& P, const FwdGroupArgs& a, hipStream_t s) 
 
 template <typename T, int M>
 hipError_t fwg_slices(const DevPlan& P, const FwdGroupArgs& a, hipStream_t s) {
-    if constexpr (sizeof(T) == 4 && M <= 2)
-        if (fwd_packed(P, DT_F32, a.B)) return fwg_detector<T, 4, M>(P, a, s);
-    return a.B > 1 ? fwg_detector<T, 2, M>(P, a, s) : fwg_detector<T, 1, M>(P, a, s);
+    switch (fwd_slices(P, sizeof(T) == 4 ? DT_F32 : DT_F64, a.B, a.nch)) {
+    case 4:
+        if constexpr (sizeof(T) == 4 && M <= 2) return fwg_detector<T, 4, M>(P, a, s);
+        return hipErrorInvalidValue;
+    case 2: return fwg_detector<T, 2, M>(P, a, s);
+    default: return fwg_detector<T, 1, M>(P, a, s);
+    }
 }
 
 template <typename T>
 hipError_t fwg_px(const DevPlan& P, const FwdGroupArgs& a, hipStream_t s) {
-    switch (fwd_px(P)) {
+    switch (line_table_px(P)) {
     case 1: return fwg_slices<T, 1>(P, a, s);
     case 2: return fwg_slices<T, 2>(P, a, s);
     case 4: return fwg_slices<T, 4>(P, a, s);

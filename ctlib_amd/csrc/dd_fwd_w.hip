@@ -15,9 +15,11 @@ namespace {
 // Work items [0, ngrp*ngx) are (slice group, 4 X-axis views) reading image rows from
 // `srcx`; the rest are Y-axis groups reading the bottom-to-top column copy.
 // fp32 variants for 512-pixel lines are held to 128 VGPRs: four waves per
-// SIMD, as many as the LDS of four 512-pixel tables per block allows.
+// SIMD, as many as the LDS of four 512-pixel tables per block allows; fp64 ones to 256 up to 20 slots.
 template <typename T, int NEM, int PPL, bool FULL>
-constexpr int fwd_w_waves() { return sizeof(T) == 4 && FULL && PPL == 8 && NEM <= 14 ? 4 : 1; }
+constexpr int fwd_w_waves() {
+    return sizeof(T) == 4 ? (FULL && PPL == 8 && NEM <= 14 ? 4 : 1) : NEM <= 20 ? 2 : 1;
+}
 
 template <typename T, int NS, int NEM, int PPL, bool FULL>
 __global__ __launch_bounds__(256, (fwd_w_waves<T, NEM, PPL, FULL>())) void k_fwd_w(DevPlan P, const T* __restrict__ srcx, const T* __restrict__ srcy,
@@ -76,11 +78,13 @@ bool all_lines(const DevPlan& P, int n) { return (P.nx == 0 || P.W == n) && (P.n
 template <typename T, int NEM, int PPL>
 hipError_t by_full(const DevPlan& P, const Args& a, hipStream_t s) {
     // Two slices share weights and addresses where that outweighs the registers of the second: fp64 data
-    // (dearer weights), lines up to 512 pixels and 895 bins, batches of pairs (fan-ED 512^2, 736 bins, B=8:
+    // (dearer weights), lines of whole lanes up to 512 pixels, up to 895 bins, batches of pairs that leave
+    // blocks for every CU's registers (fan-ED 512^2, 736 bins, B=8:
     // 1.59 -> 1.41 ms; fp32 1.38 -> 1.36, with fewer waves per SIMD, and 1024-pixel lines 5.5 -> 7.4).
     if constexpr (sizeof(T) == 8 && PPL <= 8 && NEM <= 14) {
-        if (a.B % 2 == 0 || a.B >= 9)
-            return all_lines(P, 64 * PPL) ? launch_t<T, 2, NEM, PPL, true>(P, a, s) : launch_t<T, 2, NEM, PPL, false>(P, a, s);
+        const long long blocks = (long long)((a.B + 1) / 2) * ((P.nx + 3) / 4 + (P.ny + 3) / 4) * a.nch;
+        if (all_lines(P, 64 * PPL) && (a.B % 2 == 0 || a.B >= 9) && blocks >= 2048)
+            return launch_t<T, 2, NEM, PPL, true>(P, a, s);
     }
     return all_lines(P, 64 * PPL) ? launch_t<T, 1, NEM, PPL, true>(P, a, s) : launch_t<T, 1, NEM, PPL, false>(P, a, s);
 }

@@ -110,7 +110,7 @@ __device__ __forceinline__ void fwd_group_w(const DevPlan& P, const T* __restric
         if (NS > 1)
 #pragma unroll
             for (int i = 0; i < NEM; i++) at[i] = address(i);
-        __builtin_amdgcn_sched_barrier(0);
+        if (FULL) __builtin_amdgcn_sched_barrier(0);
         // One slice's table after the other: the wave's reads of the table before were consumed
         // (in-order LDS within a wave), so it can be overwritten.
 #pragma unroll
@@ -134,20 +134,29 @@ __device__ __forceinline__ void fwd_group_w(const DevPlan& P, const T* __restric
             }
             if (lane == 0) tb[0] = make_double2(0.0, 0.0);
             if (lane == 63) tb[wtab_slot(n + 1)] = make_double2(inc, 0.0);
-            __builtin_amdgcn_sched_barrier(0);
-            // four reads under way, and no further: registers
-            constexpr int AHEAD = 4;
-            double2 ent[AHEAD];
-#pragma unroll
-            for (int i = 0; i < AHEAD && i < NEM; i++) ent[i] = *reinterpret_cast<const double2*>(NS > 1 ? at[i] : address(i));
-#pragma unroll
-            for (int i = 0; i < NEM; i++) {
-                const double2 g = ent[i % AHEAD];
-                S[q][0][i] = __builtin_fma(s, __builtin_fma(tau(i), g.y, g.x), S[q][0][i]);
-                asm volatile("" : "+v"(S[q][0][i]));
-                if (i + AHEAD < NEM)
-                    ent[i % AHEAD] = *reinterpret_cast<const double2*>(NS > 1 ? at[i + AHEAD] : address(i + AHEAD));
+            if constexpr (FULL) {
                 __builtin_amdgcn_sched_barrier(0);
+                // four reads under way, and no further: registers
+                constexpr int AHEAD = 4;
+                double2 ent[AHEAD];
+#pragma unroll
+                for (int i = 0; i < AHEAD && i < NEM; i++) ent[i] = *reinterpret_cast<const double2*>(NS > 1 ? at[i] : address(i));
+#pragma unroll
+                for (int i = 0; i < NEM; i++) {
+                    const double2 g = ent[i % AHEAD];
+                    S[q][0][i] = __builtin_fma(s, __builtin_fma(tau(i), g.y, g.x), S[q][0][i]);
+                    asm volatile("" : "+v"(S[q][0][i]));
+                    if (i + AHEAD < NEM)
+                        ent[i % AHEAD] = *reinterpret_cast<const double2*>(NS > 1 ? at[i + AHEAD] : address(i + AHEAD));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                // the bounds predicates leave the compiler's own order the faster one
+#pragma unroll
+                for (int i = 0; i < NEM; i++) {
+                    const double2 g = *reinterpret_cast<const double2*>(NS > 1 ? at[i] : address(i));
+                    S[q][0][i] = __builtin_fma(s, __builtin_fma(tau(i), g.y, g.x), S[q][0][i]);
+                }
             }
         }
     }

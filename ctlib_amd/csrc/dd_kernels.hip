@@ -222,13 +222,43 @@ int fwd_px(const DevPlan& P) {
     return m <= 2 ? 2 : m <= 4 ? 4 : m <= 8 ? 8 : 0;
 }
 
-bool fwd_packed(const DevPlan& P, int dtype, int64_t B) {
-    const int M = fwd_px(P);
-    return dtype == DT_F32 && M >= 1 && M <= 2 && (B % 4 == 0 || B % 4 == 3 || B >= 9);
+int line_table_px(const DevPlan& P) {
+    int n = P.nx ? P.W : 0;
+    if (P.ny && P.H > n) n = P.H;
+    const int m = (n + NT - 1) / NT;
+    return m <= 1 ? 1 : m <= 2 ? 2 : m <= 4 ? 4 : m <= 8 ? 8 : 0;
+}
+
+// Sharing costs 1.6 (two slices) or 2.7 (four) times a slice's block, so it pays where the blocks that
+// remain fill the chip: the candidate with the least (cost of a block) x (rounds of its waves over 16 a
+// CU), a launch below one round counting half a round and half its share.  Fan-ED 512^2: B=32 1.78 ms
+// with four slices, 2.3 with one; 96^2, 90 views, B=3: 37 us with four, 25 with one.
+int fwd_slices(const DevPlan& P, int dtype, int64_t B, int nch) {
+    const int M = line_table_px(P);
+    const int ne = edge_slots(P);
+    int best = 1;
+    double least = 0;
+    for (int NS : {1, 2, 4}) {
+        if (NS > B || (NS == 4 && (dtype != DT_F32 || M > 2))) break;
+        // tables of a part-filled group must fit the memory of B slices' own
+        if (NS == 4 && (B + 3) / 4 * 12 > B * 4) break;
+        const int waves = NS == 1 ? 4 : 8, most = NS == 4 ? 7 : NS == 2 ? 12 : 24;
+        int EH = 1;
+        while ((ne + EH - 1) / EH > most) EH *= 2;
+        const int G = waves / EH;
+        const double blocks = (double)((B + NS - 1) / NS) * ((P.nx + G - 1) / G + (P.ny + G - 1) / G) * (nch < 1 ? 1 : nch);
+        const double rounds = blocks * waves / (256.0 * 16);
+        const double cost = (NS == 1 ? 1.0 : NS == 2 ? 1.6 : 2.7) * (rounds < 1 ? 0.5 + 0.5 * rounds : rounds + 0.15) / EH;
+        if (NS == 1 || cost < least) {
+            least = cost;
+            best = NS;
+        }
+    }
+    return best;
 }
 
 size_t fwd_line_table_bytes(const DevPlan& P, int B) {
-    const int M = fwd_px(P);
+    const int M = line_table_px(P);
     if (B <= 0 || M == 0 || P.nx + P.ny == 0) return 0;
     const size_t nlt = (size_t)(P.nx ? P.H : 0) + (P.ny ? P.W : 0);
     return ((size_t)B * nlt * (NT * M + 2) + 64) * sizeof(double2);
@@ -323,7 +353,7 @@ hipError_t line_tables_t(const DevPlan& P, const void* srcx, const void* srcy, d
     const long long ntab = (long long)B * ((P.nx ? P.H : 0) + (P.ny ? P.W : 0));
     if (ntab > (1LL << 31) - 4) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((ntab + 3) / 4));
-    switch (fwd_px(P)) {
+    switch (line_table_px(P)) {
     case 1: hipLaunchKernelGGL((k_line_tables<T, 1>), grid, dim3(256), 0, s, P, (const T*)srcx, (const T*)srcy, lt, B); break;
     case 2: hipLaunchKernelGGL((k_line_tables<T, 2>), grid, dim3(256), 0, s, P, (const T*)srcx, (const T*)srcy, lt, B); break;
     case 4: hipLaunchKernelGGL((k_line_tables<T, 4>), grid, dim3(256), 0, s, P, (const T*)srcx, (const T*)srcy, lt, B); break;
@@ -336,13 +366,13 @@ hipError_t line_tables_t(const DevPlan& P, const void* srcx, const void* srcy, d
 }  // namespace
 
 hipError_t launch_line_tables(const DevPlan& P, int dtype, const void* srcx, const void* srcy, double2* ltab, int B,
-                              hipStream_t s) {
+                              int nch, hipStream_t s) {
     if (B <= 0 || P.nx + P.ny == 0) return hipSuccess;
-    if (fwd_packed(P, dtype, B)) {
+    if (fwd_slices(P, dtype, B, nch) == 4) {
         const long long nw = (long long)((B + 3) / 4) * ((P.nx ? P.H : 0) + (P.ny ? P.W : 0));
         if (nw > (1LL << 31) - 4) return hipErrorInvalidValue;
         const dim3 grid((unsigned)((nw + 3) / 4));
-        auto kern = fwd_px(P) == 1 ? k_line_tables4<1> : k_line_tables4<2>;
+        auto kern = line_table_px(P) == 1 ? k_line_tables4<1> : k_line_tables4<2>;
         hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, P, (const float*)srcx, (const float*)srcy, ltab, B);
         return hipGetLastError();
     }

@@ -44,6 +44,7 @@ struct FwdShape {                 // line->bin kernel
 // PH waves along a line (adj_shape); nch view chunks (<= 1: none)
 struct AdjShape {
     int NS, SL, PH, L;
+    int resident;  // blocks that the chip holds at once
     int nch;
 };
 // line->bin launch over prebuilt line tables (dd_fwd_group.h); tabs not null: also the residual tables
@@ -81,11 +82,12 @@ hipError_t launch_fwd(const DevPlan& P, int dtype, const void* srcx, const void*
                       const double2* ltab = nullptr);
 // Cumulative table of every image line of both axes (one wave per line) into ltab, of
 // fwd_line_table_bytes(P, B): per slice the X-axis lines (rows of srcx) then the Y-axis lines
-// (rows of srcy), 256*M + 2 entries {C_j, S_j} per line, M = fwd_px(P).  fwd_packed: per group of four
+// (rows of srcy), 256*M + 2 entries {C_j, S_j} per line, M = line_table_px(P).  Packed: per group of four
 // slices (the last slice repeated), per line the entries {C_j of slices 0, 1}, then {C_j of 2, 3}, then
 // {S_j of 0 .. 3} in fp32.
+// nch: the line chunks of the launch that reads them (fwd_slices).
 hipError_t launch_line_tables(const DevPlan& P, int dtype, const void* srcx, const void* srcy, double2* ltab, int B,
-                              hipStream_t s);
+                              int nch, hipStream_t s);
 hipError_t launch_fwd_lt_f32(const DevPlan& P, const FwdGroupArgs& a, hipStream_t s);
 hipError_t launch_fwd_lt_f64(const DevPlan& P, const FwdGroupArgs& a, hipStream_t s);
 // out[i] = sum_k parts[k*count + i], k < nch (out may equal parts)
@@ -93,13 +95,17 @@ hipError_t launch_sum_parts(void* out, const void* parts, int dtype, int nch, si
 size_t fwd_lds_bytes(const DevPlan& P, bool weighted, int G);
 // Pixels per thread M of the line -> bin launch (lines of at most 256*M pixels; 0: too long).
 int fwd_px(const DevPlan& P);
-// Whether the line tables of a batch are packed by four slices (dd_fwd_group.h): fp32 data, lines up to
-// 512 pixels (a CU holds the buffers of only one block of packed longer ones: fan-ED 1024^2 B=4 2.15 ms
-// against 2.07 in pairs), and few enough slots of the last group empty that it pays - a packed group of four costs
-// 1.6 pairs (they also need no more memory then: 48 bytes an entry and group against 16 and slice).
-bool fwd_packed(const DevPlan& P, int dtype, int64_t B);
-// Bytes of the prebuilt line tables of a batch of B (an upper bound where they are packed): (B * (lines of both axes) * (256*M + 2) + 64) * 16,
-// the last 64 entries because the line -> bin kernel copies whole chunks of 64.
+// Pixels per thread M of the prebuilt line tables (lines of at most 256*M pixels; 0: too long).
+int line_table_px(const DevPlan& P);
+// Slots of 64 bin edges of a view: detectors of whole slots have their edge D taken apart.
+inline bool whole_slots(const DevPlan& P) { return P.D == 512 || P.D == 1024 || P.D == 1536; }
+inline int edge_slots(const DevPlan& P) { return whole_slots(P) ? P.D / 64 : (P.D + 1 + 63) / 64; }
+// Slices that a block of the line -> bin kernel over prebuilt tables holds: 1, 2, or 4 with the line tables
+// packed by four slices (fp32 data, lines up to 512 pixels; a CU holds the buffers of only one block of
+// packed longer ones: fan-ED 1024^2 B=4 2.15 ms against 2.07 in pairs).
+int fwd_slices(const DevPlan& P, int dtype, int64_t B, int nch);
+// Bytes of the prebuilt line tables of a batch of B, (B * (lines of both axes) * (256*M + 2) + 64) * 16;
+// packed tables (48 bytes an entry for a group of four) are chosen only where they fit in it.
 size_t fwd_line_table_bytes(const DevPlan& P, int B);
 
 // projection fused with the residual bin tables of projection_t: writes y = A x (y may be null)
@@ -132,9 +138,8 @@ hipError_t launch_adj(const DevPlan& P, int dtype, const double2* tabs, void* ou
                       bool weighted, double wscale, AdjShape shape, hipStream_t s);
 // Launch shape of launch_adj for a batch of B, without the view chunks (nch = 1).
 AdjShape adj_shape(const DevPlan& P, int dtype, bool weighted, int64_t B);
-// Its work items (slice groups x line tiles of both axes), and the blocks the chip holds at once.
+// Its work items (slice groups x line tiles of both axes).
 int64_t adj_items(const DevPlan& P, const AdjShape& sh, int64_t B);
-int adj_resident(const AdjShape& sh);
 // Image lines that the view chunks are counted in (abi.cpp adj_chunks).
 int adj_tile_lines(const DevPlan& P);
 hipError_t launch_adj_f32(const DevPlan& P, const AdjArgs& a, hipStream_t s);
